@@ -15,42 +15,105 @@ void batch_inverse_m31(const uint32_t* src, uint32_t* dst, uint64_t n);  // batc
 
 namespace tw {
 
-__host__ __device__ inline pt pdouble_n(pt p, uint32_t n) {
-  for (uint32_t i = 0; i < n; i++) p = pmul(p, p);
-  return p;
-}
-__device__ inline pt ppow(pt p, uint32_t e) {
-  pt r = {1, 0};
-  while (e) {
-    if (e & 1) r = pmul(r, p);
-    p = pmul(p, p);
-    e >>= 1;
+// Level 0 holds the x of initial + step * brev(i): bit b of i contributes the fixed point
+// weight[b] = step * 2^(half_log - 1 - b), so a thread multiplies the weights of its set bits
+// and then takes its 16 values from one product each with 16 uniform points.  The level above
+// needs no points: brev(2i) over one more bit is brev(i), so entry i of level j + 1 is the
+// doubling x -> 2x^2 - 1 of entry 2i of level j, and a block that owns 2^12 consecutive values
+// of level 0 owns 2^11 of level 1, ... , one of level 12, and, where its index is a multiple of
+// 2^z, one of levels 12 + 1 .. 12 + z.  Bound by the latency of the products and of the
+// doublings (2^22: 103 -> 13.8 us against a full power of the step per entry, which took 2 x 31
+// products each; the stores alone take 3 us).
+constexpr uint32_t TREE_BLOCK_LOG = 12, TREE_NT = 256;
+
+struct TreeArgs {
+  pt initial;
+  pt weight[30];  // identity from half_log on
+  pt lane16[16];  // sum of the weights of bits 0, 1, 10, 11 selected by the index's bits
+};
+
+__global__ __launch_bounds__(TREE_NT) void tree_kernel(uint32_t* __restrict__ out, TreeArgs A, uint32_t log_size) {
+  const uint32_t size = 1u << log_size, half_log = log_size - 1, half = size >> 1;  // log_size >= 1
+  const uint32_t t = threadIdx.x, blk = blockIdx.x;
+  if (blk == 0 && t == 0) out[size - 1] = 1;
+  pt q = A.initial;
+  for (uint32_t b = TREE_BLOCK_LOG; b < half_log; b++)  // uniform
+    if ((blk >> (b - TREE_BLOCK_LOG)) & 1) q = pmul(q, A.weight[b]);
+#pragma unroll
+  for (int b = 0; b < 8; b++) {
+    const pt r = pmul(q, A.weight[b + 2]);
+    if ((t >> b) & 1) q = r;
   }
-  return r;
+  // value c of group k: index i = blk 2^12 + 2^10 k + 4 t + c
+  uint32_t x[4][4];
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) x[k][c] = pmul(q, A.lane16[4 * k + c]).x;
+  auto twice = [](uint32_t v) { return sub(canon(2 * sqr(v)), 1); };
+  // level j starts at size - (size >> j); j <= 2: 4, 2, 1 values per thread and group
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const uint32_t i = (blk << TREE_BLOCK_LOG) + (k << 10) + 4 * t;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      uint32_t* lvl = out + (size - (size >> j));
+#pragma unroll
+      for (int c = 0; c < (4 >> j); c++)
+        if (i + ((uint32_t)c << j) < half && log_size > (uint32_t)j) lvl[(i >> j) + c] = x[k][c];
+#pragma unroll
+      for (int c = 0; c < (4 >> (j + 1)); c++) x[k][c] = twice(x[k][2 * c]);
+      if (j == 2) x[k][0] = twice(x[k][0]);
+    }
+  }
+#pragma unroll 1
+  for (uint32_t j = 3; j < 10; j++) {
+    if (j >= log_size) return;  // uniform
+    uint32_t* lvl = out + (size - (size >> j));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t i = (blk << TREE_BLOCK_LOG) + (k << 10) + 4 * t;
+      if ((t & ((1u << (j - 2)) - 1)) == 0 && i < half) lvl[i >> j] = x[k][0];
+      x[k][0] = twice(x[k][0]);
+    }
+  }
+  if (t) return;
+  // levels 10 .. : the block's values 2^10 k, then its first value alone
+#pragma unroll 1
+  for (uint32_t j = 10; j < log_size; j++) {
+    uint32_t* lvl = out + (size - (size >> j));
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint32_t i = (blk << TREE_BLOCK_LOG) + (k << 10);
+      if ((i & ((1u << j) - 1)) == 0 && i < half) lvl[i >> j] = x[k][0];
+      x[k][0] = twice(x[k][0]);
+    }
+    if (j >= TREE_BLOCK_LOG && (blk & ((2u << (j - TREE_BLOCK_LOG)) - 1))) return;
+  }
 }
 
-__global__ void tree_kernel(uint32_t* out, pt initial, pt step, uint32_t log_size) {
-  const uint32_t size = 1u << log_size;
-  uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= size) return;
-  if (t == size - 1) {
-    out[t] = 1;
-    return;
-  }
-  // level j occupies [size - (size >> j), size - (size >> (j + 1)))
-  uint32_t j = 0;
-  while (t >= size - (size >> (j + 1))) j++;
-  uint32_t i = t - (size - (size >> j));
-  uint32_t lvl_log = log_size - j;  // coset log size at this level
-  pt ini = pdouble_n(initial, j), st = pdouble_n(step, j);
-  out[t] = pmul(ini, ppow(st, brev(i, lvl_log - 1))).x;
-}
+__global__ void one_kernel(uint32_t* out) { out[0] = 1; }
 
 void compute_tree(uint32_t* out, pt initial, pt step, uint32_t log_size) {
-  uint32_t size = 1u << log_size;
-  timed("twiddle_tree", [&] {
-    tree_kernel<<<ceil_div(size, 256), 256, 0, ctx().cur>>>(out, initial, step, log_size);
-  });
+  if (log_size == 0) {  // a coset of one point: the trailing 1 alone
+    timed("twiddle_tree", [&] { one_kernel<<<1, 1, 0, ctx().cur>>>(out); });
+    return;
+  }
+  TreeArgs A;
+  A.initial = initial;
+  const uint32_t half_log = log_size - 1;
+  pt w = step;
+  for (uint32_t b = 0; b < 30; b++) A.weight[b] = pt{1, 0};
+  for (uint32_t b = half_log; b-- > 0; w = pmul(w, w)) A.weight[b] = w;  // weight[half_log - 1] = step
+  for (uint32_t s = 0; s < 16; s++) {
+    const uint32_t bit[4] = {0, 1, 10, 11};
+    pt r = {1, 0};
+    for (int b = 0; b < 4; b++)
+      if ((s >> b) & 1) r = pmul(r, A.weight[bit[b]]);
+    A.lane16[s] = r;
+  }
+  const uint32_t blocks = half_log > TREE_BLOCK_LOG ? 1u << (half_log - TREE_BLOCK_LOG) : 1u;
+  timed("twiddle_tree", [&] { tree_kernel<<<blocks, TREE_NT, 0, ctx().cur>>>(out, A, log_size); });
 }
 
 }  // namespace tw
