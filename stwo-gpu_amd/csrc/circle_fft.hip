@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "fft.hpp"
+#include "fft_matrix.hpp"
 #include "field.hpp"
 #include "gmem.hpp"
 #include "runtime.hpp"
@@ -720,17 +721,41 @@ static void launch_pass(const PassPlan& p, const PassArgs& base) {
   });
 }
 
+// the matrix-core kernels for small columns take blowups 1 .. 8
+static bool use_matrices_evaluate(uint32_t src_log, uint32_t log_n, uint64_t n_cols) {
+  return src_log + 3 >= log_n && use_matrices_tile(log_n, n_cols);
+}
+// Device memory for the matrices of a transform of whole small columns (0: none are used).
+static size_t tile_workspace_bytes(uint32_t log_n, uint64_t n_cols) {
+  return use_matrices_tile(log_n, n_cols) ? tile_matrix_bytes(log_n) : 0;
+}
+// The matrices of a transform of n_cols whole columns over the domain of log_n, when it uses
+// them: enqueued before the pointer tables are uploaded, so they are made while the host copies.
+static DevBuf tile_workspace(bool inverse, bool used, uint32_t log_n, const uint32_t* tw, uint64_t tree_len) {
+  if (!used || tree_len < (1ull << (log_n - 1))) return DevBuf();  // (a short tree is refused later)
+  DevBuf ws(tile_matrix_bytes(log_n));
+  tile_matrices(inverse, log_n, tw + (tree_len - (1ull << (log_n - 1))), ws.as<unsigned char>());
+  return ws;
+}
+
 // Inverse FFT of n_cols columns of one log size (device pointer tables): the first pass
 // reads d_src, every pass writes d_cols (d_src == d_cols: in place).
+// ws: tile_workspace_bytes of device memory (may be null where that is 0), where the matrices
+// are already when ws_filled.
 void interpolate_same_size(uint32_t* const* d_cols, uint32_t n_cols, uint32_t log_n, const uint32_t* itw,
-                           uint64_t tree_len, const uint32_t* const* d_src = nullptr, uint32_t kc = 0) {
-  if (!d_src) d_src = (const uint32_t* const*)d_cols;
+                           uint64_t tree_len, const uint32_t* const* d_src, uint32_t kc, void* ws, bool ws_filled = false) {
   require(log_n >= 1 && log_n <= 30, "interpolate: log size out of range");
   require(tree_len >= (1ull << (log_n - 1)), "interpolate: twiddle tree smaller than the domain");
   if (log_n <= 2) {
     timed("fft_tiny_inv", [&] {
       fft_tiny_kernel<true><<<ceil_div(n_cols, 64), 64, 0, ctx().cur>>>(d_cols, d_src, n_cols, log_n, log_n);
     });
+    return;
+  }
+  if (use_matrices_tile(log_n, n_cols)) {
+    const uint32_t* t = itw + (tree_len - (1ull << (log_n - 1)));
+    if (!ws_filled) tile_matrices(true, log_n, t, (unsigned char*)ws);
+    interpolate_tiles(d_src, d_cols, n_cols, log_n, t, (unsigned char*)ws);
     return;
   }
   PassArgs A{};
@@ -752,13 +777,20 @@ void interpolate_same_size(uint32_t* const* d_cols, uint32_t n_cols, uint32_t lo
 // Forward FFT: src columns (2^src_log coefficients) evaluated on the canonic domain
 // of log_n >= src_log, written to dst (device pointer tables).
 void evaluate_same_size(uint32_t* const* d_dst, const uint32_t* const* d_src, uint32_t n_cols, uint32_t src_log,
-                        uint32_t log_n, const uint32_t* tw, uint64_t tree_len, uint32_t kc = 0) {
+                        uint32_t log_n, const uint32_t* tw, uint64_t tree_len, uint32_t kc, void* ws,
+                        bool ws_filled = false) {
   require(log_n >= 1 && log_n <= 30 && src_log <= log_n, "evaluate: log sizes out of range");
   require(tree_len >= (1ull << (log_n - 1)), "evaluate: twiddle tree smaller than the domain");
   if (log_n <= 2) {
     timed("fft_tiny_fwd", [&] {
       fft_tiny_kernel<false><<<ceil_div(n_cols, 64), 64, 0, ctx().cur>>>(d_dst, d_src, n_cols, log_n, src_log);
     });
+    return;
+  }
+  if (use_matrices_evaluate(src_log, log_n, n_cols)) {
+    const uint32_t* t = tw + (tree_len - (1ull << (log_n - 1)));
+    if (!ws_filled) tile_matrices(false, log_n, t, (unsigned char*)ws);
+    evaluate_tiles(d_src, d_dst, n_cols, src_log, log_n, t, (unsigned char*)ws);
     return;
   }
   PassArgs A{};
@@ -788,19 +820,29 @@ static void launch_lde_strided(uint32_t blocks, const PassArgs& Ai, const PassAr
   }
 }
 
+size_t lde_workspace_bytes(uint32_t n, uint32_t log_blowup, uint64_t n_cols, LdeVariant var) {
+  if (var.mat && n >= 17 && n <= 20) return lde_matrix_bytes(n, log_blowup);
+  return std::max(tile_workspace_bytes(n, n_cols), tile_workspace_bytes(n + log_blowup, n_cols));
+}
+
 // Interpolate d_src (2^n evaluations) into d_coeffs and evaluate on the canonic domain of
 // log n + log_blowup into d_lde.  d_src may equal d_coeffs.
 void lde_same_size(const uint32_t* const* d_src, uint32_t* const* d_coeffs, uint32_t* const* d_lde, uint32_t n_cols,
                    uint32_t n, uint32_t log_blowup, const uint32_t* tw, const uint32_t* itw, uint64_t tree_len,
-                   LdeVariant var) {
+                   LdeVariant var, void* ws) {
   const uint32_t m = n + log_blowup;
   require(m <= 30, "lde: log size out of range");
   require(tree_len >= (1ull << (m - 1)), "lde: twiddle tree smaller than the evaluation domain");
+  if (var.mat && n >= 17 && n <= 20) {
+    lde_matrices(d_src, d_coeffs, d_lde, n_cols, n, log_blowup, tw + (tree_len - (1ull << (m - 1))),
+                 itw + (tree_len - (1ull << (n - 1))), (unsigned char*)ws);
+    return;
+  }
   if (!var.fused || n < 14 || n > 12 + KS_MAX) {
     const uint32_t kci = (var.kc == 13 && n >= 14 && n - 13 <= KS_MAX) ? 13 : 0;
     const uint32_t kcf = (var.kc == 13 && m >= 14 && m - 13 <= KS_MAX) ? 13 : 0;
-    interpolate_same_size(d_coeffs, n_cols, n, itw, tree_len, d_src, kci);
-    evaluate_same_size(d_lde, (const uint32_t* const*)d_coeffs, n_cols, n, m, tw, tree_len, kcf);
+    interpolate_same_size(d_coeffs, n_cols, n, itw, tree_len, d_src, kci, ws);
+    evaluate_same_size(d_lde, (const uint32_t* const*)d_coeffs, n_cols, n, m, tw, tree_len, kcf, ws);
     return;
   }
   const uint32_t k = n - 12, t = (k <= 8 ? 13 : BS_LDE) - k;
@@ -865,24 +907,31 @@ void lde_mixed(const uint32_t* const* src, uint32_t* const* coeffs, uint32_t* co
     }
     DevBuf d = upload(t.data(), t.size() * sizeof(void*));
     const void* const* base = d.as<const void*>();
+    const LdeVariant var = lde_variant_for(kv.first, log_blowup, cnt);
+    const size_t wb = lde_workspace_bytes(kv.first, log_blowup, cnt, var);
+    DevBuf ws = wb ? DevBuf(wb) : DevBuf();
     lde_same_size((const uint32_t* const*)base, (uint32_t* const*)(base + cnt), (uint32_t* const*)(base + 2 * cnt),
-                  (uint32_t)cnt, kv.first, log_blowup, tw, itw, tree_len, lde_variant_for(kv.first, log_blowup, cnt));
+                  (uint32_t)cnt, kv.first, log_blowup, tw, itw, tree_len, var, ws.p);
   }
+}
+
+// Columns of one size (the common case, e.g. 2^16 columns of one trace): the caller's pointer
+// table is uploaded as it is, once when the columns are transformed in place.
+static void interpolate_one_size(uint32_t* const* cols, uint32_t n_cols, uint32_t log_n, const uint32_t* itw,
+                                 uint64_t tree_len, const uint32_t* const* src) {
+  DevBuf ws = tile_workspace(true, use_matrices_tile(log_n, n_cols), log_n, itw, tree_len);
+  DevBuf table = upload(cols, (size_t)n_cols * sizeof(void*));
+  DevBuf stable = src ? upload(src, (size_t)n_cols * sizeof(void*)) : DevBuf();
+  interpolate_same_size(table.as<uint32_t*>(), n_cols, log_n, itw, tree_len,
+                        src ? stable.as<const uint32_t*>() : table.as<const uint32_t*>(), 0, ws.p, true);
 }
 
 // Group columns by size and run each class.  cols/logs are host arrays; src (optional)
 // holds the inputs when they are not transformed in place.
 void interpolate_mixed(uint32_t* const* cols, const uint32_t* logs, uint32_t n_cols, const uint32_t* itw,
                        uint64_t tree_len, const uint32_t* const* src = nullptr) {
-  // one size (the common case, e.g. 2^16 columns of one trace): the caller's pointer table
-  // is uploaded as it is, once when the columns are transformed in place
-  if (n_cols && std::all_of(logs, logs + n_cols, [&](uint32_t l) { return l == logs[0]; })) {
-    DevBuf table = upload(cols, (size_t)n_cols * sizeof(void*));
-    DevBuf stable = src ? upload(src, (size_t)n_cols * sizeof(void*)) : DevBuf();
-    interpolate_same_size(table.as<uint32_t*>(), n_cols, logs[0], itw, tree_len,
-                          src ? stable.as<const uint32_t*>() : table.as<const uint32_t*>());
-    return;
-  }
+  if (n_cols && std::all_of(logs, logs + n_cols, [&](uint32_t l) { return l == logs[0]; }))
+    return interpolate_one_size(cols, n_cols, logs[0], itw, tree_len, src);
   std::map<uint32_t, std::pair<std::vector<uint32_t*>, std::vector<const uint32_t*>>> by;
   for (uint32_t i = 0; i < n_cols; i++) {
     by[logs[i]].first.push_back(cols[i]);
@@ -892,8 +941,9 @@ void interpolate_mixed(uint32_t* const* cols, const uint32_t* logs, uint32_t n_c
     size_t n = kv.second.first.size();
     DevBuf table = upload(kv.second.first.data(), n * sizeof(void*));
     DevBuf stable = upload(kv.second.second.data(), n * sizeof(void*));
+    DevBuf ws = tile_workspace(true, use_matrices_tile(kv.first, n), kv.first, itw, tree_len);
     interpolate_same_size(table.as<uint32_t*>(), (uint32_t)n, kv.first, itw, tree_len,
-                          stable.as<const uint32_t*>());
+                          stable.as<const uint32_t*>(), 0, ws.p, true);
   }
 }
 void evaluate_mixed(const uint32_t* const* src, const uint32_t* src_logs, uint32_t* const* dst,
@@ -903,10 +953,11 @@ void evaluate_mixed(const uint32_t* const* src, const uint32_t* src_logs, uint32
   if (n_cols && std::all_of(src_logs, src_logs + n_cols, [&](uint32_t l) { return l == src_logs[0]; }) &&
       std::all_of(dst_logs, dst_logs + n_cols, [&](uint32_t l) { return l == dst_logs[0]; })) {
     const bool in_place = std::equal(src, src + n_cols, (const uint32_t* const*)dst);
+    DevBuf ws = tile_workspace(false, use_matrices_evaluate(src_logs[0], dst_logs[0], n_cols), dst_logs[0], tw, tree_len);
     DevBuf td = upload(dst, (size_t)n_cols * sizeof(void*));
     DevBuf ts = in_place ? DevBuf() : upload(src, (size_t)n_cols * sizeof(void*));
     evaluate_same_size(td.as<uint32_t*>(), in_place ? td.as<const uint32_t*>() : ts.as<const uint32_t*>(), n_cols,
-                       src_logs[0], dst_logs[0], tw, tree_len);
+                       src_logs[0], dst_logs[0], tw, tree_len, 0, ws.p, true);
     return;
   }
   std::map<std::pair<uint32_t, uint32_t>, std::pair<std::vector<const uint32_t*>, std::vector<uint32_t*>>> by;
@@ -919,8 +970,9 @@ void evaluate_mixed(const uint32_t* const* src, const uint32_t* src_logs, uint32
     size_t n = kv.second.first.size();
     DevBuf ts = upload(kv.second.first.data(), n * sizeof(void*));
     DevBuf td = upload(kv.second.second.data(), n * sizeof(void*));
+    DevBuf ws = tile_workspace(false, use_matrices_evaluate(kv.first.first, kv.first.second, n), kv.first.second, tw, tree_len);
     evaluate_same_size(td.as<uint32_t*>(), ts.as<const uint32_t*>(), (uint32_t)n, kv.first.first, kv.first.second,
-                       tw, tree_len);
+                       tw, tree_len, 0, ws.p, true);
   }
 }
 
@@ -949,8 +1001,8 @@ extern "C" void interpolate_columns(uint32_t eval_domain_size, uint32_t* const* 
   guarded([&] {
     if (!values_size) return;
     require(is_pow2(number_of_rows) && number_of_rows == 2ull * eval_domain_size, "interpolate_columns: bad sizes");
-    std::vector<uint32_t> logs(values_size, log2_exact(number_of_rows));
-    fft::interpolate_mixed(values, logs.data(), values_size, inverse_twiddles_tree, inverse_twiddle_tree_size);
+    fft::interpolate_one_size(values, values_size, log2_exact(number_of_rows), inverse_twiddles_tree,
+                              inverse_twiddle_tree_size, nullptr);
     sync();
   });
 }

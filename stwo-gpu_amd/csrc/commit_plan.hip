@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "fft.hpp"
+#include "fft_matrix.hpp"
 #include "merkle_plan.hpp"
 #include "runtime.hpp"
 
@@ -40,6 +41,7 @@ LdeVariant lde_variant_for(uint32_t n, uint32_t log_blowup, uint64_t n_cols) {
   // strided layers, log sizes 14..20), measured faster than separate strided passes there
   LdeVariant v;
   v.fused = n >= 14 && n <= 20;
+  v.mat = use_matrices_lde(n, log_blowup, n_cols);
   return v;
 }
 void set_lde_variant(uint32_t n, uint32_t log_blowup, uint64_t n_cols, LdeVariant v) {
@@ -53,6 +55,7 @@ struct CommitPlan {
     uint32_t log, n;
     DevBuf tables;  // [src | coeffs | lde] device pointer tables
     fft::LdeVariant var;
+    DevBuf ws;  // lde_workspace_bytes for var
   };
   std::vector<Class> classes;
   uint32_t log_blowup;
@@ -67,7 +70,13 @@ struct CommitPlan {
   void enqueue_class(const Class& c) const {
     const void* const* base = c.tables.as<const void*>();
     fft::lde_same_size((const uint32_t* const*)base, (uint32_t* const*)(base + c.n),
-                       (uint32_t* const*)(base + 2 * c.n), c.n, c.log, log_blowup, tw, itw, tree_len, c.var);
+                       (uint32_t* const*)(base + 2 * c.n), c.n, c.log, log_blowup, tw, itw, tree_len, c.var, c.ws.p);
+  }
+
+  void set_variant(Class& c, fft::LdeVariant v) const {
+    c.var = v;
+    const size_t b = fft::lde_workspace_bytes(c.log, log_blowup, c.n, v);
+    c.ws = b ? DevBuf(b) : DevBuf();
   }
 
   // Classes run on the auxiliary streams, largest first, round robin; each records an
@@ -141,11 +150,13 @@ struct CommitPlan {
       std::vector<fft::LdeVariant> cand = {{12, false}};
       if (c.log - 13 <= 9 && c.log + log_blowup - 13 <= 9) cand.push_back({13, false});
       if (c.log <= 21) cand.push_back({12, true});
+      // the matrix-core passes are tried from half the columns that they are the default for
+      if (fft::use_matrices_lde(c.log, log_blowup, 2ull * c.n)) cand.push_back({12, true, true});
       if (cand.size() == 1) continue;
       float best = 1e30f;
       fft::LdeVariant best_v = cand[0];
       for (const auto& v : cand) {
-        c.var = v;
+        set_variant(c, v);
         enqueue_class(c);  // warm-up
         float ms_min = 1e30f;
         for (int rep = 0; rep < 3; rep++) {
@@ -162,7 +173,7 @@ struct CommitPlan {
           best_v = v;
         }
       }
-      c.var = best_v;
+      set_variant(c, best_v);
       fft::set_lde_variant(c.log, log_blowup, c.n, best_v);
     }
     // graph replay against stream launches of the whole plan (a plan of many size classes
@@ -232,8 +243,8 @@ extern "C" int stwo_hip_commit_plan_create(StwoCommitPlan** out, uint32_t n_cols
         t[n + i] = coeffs[kv.second[i]];
         t[2 * n + i] = ldes[kv.second[i]];
       }
-      CommitPlan::Class c{kv.first, n, upload(t.data(), t.size() * sizeof(void*)),
-                          fft::lde_variant_for(kv.first, log_blowup, n)};
+      CommitPlan::Class c{kv.first, n, upload(t.data(), t.size() * sizeof(void*)), {}, DevBuf()};
+      p.set_variant(c, fft::lde_variant_for(kv.first, log_blowup, n));
       p.classes.push_back(std::move(c));
     }
     p.class_done.resize(p.classes.size());

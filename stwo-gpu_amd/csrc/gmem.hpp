@@ -75,6 +75,29 @@ struct BufCol {
   __device__ __forceinline__ void store(uint32_t v, uint32_t i, uint32_t s) const {
     __builtin_amdgcn_raw_buffer_store_b32(v, rs, i * 4u, s * 4u, 0);
   }
+  // words i + s .. i + s + 3.  NT: a streaming access (nontemporal hint), for buffers larger than
+  // the caches that pass through once
+  template <bool NT = false>
+  __device__ __forceinline__ uint4 load4(uint32_t i, uint32_t s) const {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, i * 4u, s * 4u, NT ? 2 : 0);
+    return make_uint4(v[0], v[1], v[2], v[3]);
+  }
+  template <bool NT = false>
+  __device__ __forceinline__ void store4(uint4 v, uint32_t i, uint32_t s) const {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    __builtin_amdgcn_raw_buffer_store_b128(u32x4{v.x, v.y, v.z, v.w}, rs, i * 4u, s * 4u, NT ? 2 : 0);
+  }
+  // words i + s and i + s + 1
+  template <bool NT = false>
+  __device__ __forceinline__ uint2 load2(uint32_t i, uint32_t s) const {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(rs, i * 4u, s * 4u, NT ? 2 : 0);
+    return make_uint2(v[0], v[1]);
+  }
+  template <bool NT = false>
+  __device__ __forceinline__ void store2(uint32_t v0, uint32_t v1, uint32_t i, uint32_t s) const {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{v0, v1}, rs, i * 4u, s * 4u, NT ? 2 : 0);
+  }
 };
 
 }  // namespace sh

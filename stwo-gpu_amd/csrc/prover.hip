@@ -381,12 +381,25 @@ uint32_t half_step(uint32_t log) { return (1u << (32 - log)) & 0x7fffffffu; }
 
 }  // namespace
 
+// schedules of a batch's two extensions (trace, composition), and the device memory that the
+// larger of them needs
+struct LdePlans {
+  fft::LdeVariant t, q;
+  size_t ws;
+  LdePlans(const Params& p, uint32_t n_jobs)
+      : t(fft::lde_variant_for(p.log_n, 1, (uint64_t)n_jobs * p.n_cols)),
+        q(fft::lde_variant_for(p.log_n + 1, 1, 4ull * n_jobs)),
+        ws(std::max(fft::lde_workspace_bytes(p.log_n, 1, (uint64_t)n_jobs * p.n_cols, t),
+                    fft::lde_workspace_bytes(p.log_n + 1, 1, 4ull * n_jobs, q))) {}
+};
+
 // byte stride between the arenas of a batch's jobs
 uint64_t job_stride(const Params& p, const Layout& L) { return (Arena(p, L).end + 4095) & ~4095ull; }
 
 uint64_t footprint_bytes(const Params& p, uint32_t n_jobs) {
   Layout L(p);
-  return job_stride(p, L) * n_jobs + 64 * 1024 * (uint64_t)(3 + L.n_line) +  // plus plan tables
+  return job_stride(p, L) * n_jobs + LdePlans(p, n_jobs).ws +
+         64 * 1024 * (uint64_t)(3 + L.n_line) +  // plus plan tables
          (uint64_t)n_jobs * 16 * ((uint64_t)p.n_cols + 4);                      // batch pointer tables
 }
 
@@ -408,6 +421,10 @@ Job::Job(const Params& p_, hipStream_t s, uint32_t n_jobs_)
   Arena A(p, L);
   jstride = n_jobs > 1 ? job_stride(p, L) : 0;
   arena = DevBuf(n_jobs > 1 ? jstride * n_jobs : A.end);
+  const LdePlans lde_plans(p, n_jobs);
+  var_t = lde_plans.t;
+  var_q = lde_plans.q;
+  if (lde_plans.ws) fft_ws = DevBuf(lde_plans.ws);
   char* base = arena.as<char>();
   coeffs = (uint32_t*)(base + A.coeffs);
   lde = (uint32_t*)(base + A.lde);
@@ -565,6 +582,7 @@ Job::~Job() {
   tree_q.reset();
   tree_l.clear();
   tables_ = DevBuf();
+  fft_ws = DevBuf();
   arena = DevBuf();
 }
 
@@ -579,7 +597,7 @@ void Job::enqueue(const uint64_t* seeds) {
   timed("channel_begin", [&] { k_begin<<<one, 1, 0, stream>>>(jb, sd, p, L.n_line, js); });
   wide_fib_trace_async((uint32_t* const*)t_coeffs, C, ln, &jb->seed, K, js);
   fft::lde_same_size(b_coeffs, (uint32_t* const*)b_coeffs, (uint32_t* const*)b_lde, K * C, ln, 1, tw, itw, tree_len,
-                     fft::lde_variant_for(ln, 1, (uint64_t)K * C));
+                     var_t, fft_ws.p);
   {
     const merkle::RootDraw rd{&jb->ch, &jb->alpha, 0};
     if (!tree_t->enqueue(nullptr, &rd))
@@ -592,7 +610,7 @@ void Job::enqueue(const uint64_t* seeds) {
   uint32_t* q4[4] = {comp, comp + cs(2 * n), comp + 2 * cs(2 * n), comp + 3 * cs(2 * n)};
   wide_fib_quotients_async(q4, t_lde, powers, dinv, (uint32_t)(2 * n), C, K, js);
   fft::lde_same_size(b_comp, (uint32_t* const*)b_comp, (uint32_t* const*)b_comp_lde, 4 * K, ln + 1, 1, tw, itw,
-                     tree_len, fft::lde_variant_for(ln + 1, 1, 4ull * K));
+                     tree_len, var_q, fft_ws.p);
   {
     const merkle::RootDraw rd{&jb->ch, jb->z, 1};
     if (!tree_q->enqueue(nullptr, &rd))

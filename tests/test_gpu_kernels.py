@@ -18,3 +18,67 @@ def test_twiddle_tree_levels(log_n, start):
     tw, itw = O.precompute_twiddles(c.initial_index, c.step_size, c.log_size)
     assert (tree.twiddles.to_numpy() == tw).all()
     assert (tree.itwiddles.to_numpy() == itw).all()
+
+
+def _m31(rng, n):
+    """Uniform values with the extremes among them."""
+    v = rng.integers(0, S.P, n, dtype=np.uint32)
+    v[:: max(1, n // 7)] = S.P - 1
+    v[1 :: max(1, n // 5)] = 0
+    return v
+
+
+@pytest.mark.parametrize("log_n,n_cols,blowup", [(10, (1 << 14) + 1, 0), (10, (1 << 12) + 3, 2), (10, 8197, 1),
+                                                 (11, 8193, 0), (11, 4099, 1), (12, 4097, 0), (9, 4098, 3),
+                                                 (9, 16387, 1), (8, 16385, 2), (10, 16386, 3)])
+def test_small_columns_on_matrix_cores(log_n, n_cols, blowup):
+    """Batches of small columns large enough for the matrix cores: the number of columns leaves the
+    last group partly empty, and columns of the extreme values lie at both ends."""
+    rng = np.random.default_rng(log_n * 1000 + n_cols)
+    m = log_n + blowup
+    picks = [0, 1, 2, 3, n_cols // 2, n_cols - 2, n_cols - 1]
+    host = rng.integers(0, S.P, (n_cols, 1 << log_n), dtype=np.uint32)
+    host[1][:] = S.P - 1
+    host[2][:] = 0
+    host[n_cols - 1][::2] = S.P - 1
+    src = S.BaseFieldVec.from_numpy(host.reshape(-1))
+    dst = S.BaseFieldVec.uninitialized(n_cols << m)
+    coset = S.canonic_half_coset(m)
+    tw, itw = S.cached_twiddles(coset)
+    sp = S._ptr_array([src.ptr + (c << (log_n + 2)) for c in range(n_cols)])
+    dp = S._ptr_array([dst.ptr + (c << (m + 2)) for c in range(n_cols)])
+    lo, lm = np.full(n_cols, log_n, np.uint32), np.full(n_cols, m, np.uint32)
+    L = S.lib()
+    S.check(L.stwo_hip_evaluate_columns_async(sp, lo.ctypes.data_as(S.u32p), dp, lm.ctypes.data_as(S.u32p), n_cols,
+                                              tw, 1 << coset.log_size))
+    S.check(L.stwo_hip_interpolate_columns_async(sp, lo.ctypes.data_as(S.u32p), n_cols, itw, 1 << coset.log_size))
+    out, back = dst.to_numpy().reshape(n_cols, -1), src.to_numpy().reshape(n_cols, -1)
+    otw, oitw = O.precompute_twiddles(coset.initial_index, coset.step_size, coset.log_size)
+    half = S.canonic_half_coset(log_n).initial_index
+    for c in picks:
+        ext = np.zeros(1 << m, np.uint32)
+        ext[: 1 << log_n] = host[c]
+        assert (out[c] == O.evaluate(ext, coset.initial_index, otw)).all(), c
+        assert (back[c] == O.interpolate(host[c], half, oitw)).all(), c
+
+
+@pytest.mark.parametrize("log_n,n_cols,blowup", [(17, 385, 1), (18, 193, 1), (19, 97, 1), (20, 49, 1), (18, 193, 2),
+                                                 (17, 384, 3)])
+def test_extension_on_matrix_cores(log_n, n_cols, blowup):
+    """Every number of strided layers (5 .. 8) of the matrix-core extension, at the fewest columns
+    that take it and one more than a whole group."""
+    rng = np.random.default_rng(log_n + n_cols)
+    m = log_n + blowup
+    host = {c: rng.integers(0, S.P, 1 << log_n, dtype=np.uint32) for c in (0, 1, n_cols // 2, n_cols - 1)}
+    host[1][:] = S.P - 1
+    cols = [S.BaseFieldVec.from_numpy(host[c]) if c in host else S.BaseFieldVec.zeros(1 << log_n) for c in range(n_cols)]
+    coset = S.canonic_half_coset(m)
+    tw, itw = S.cached_twiddles(coset)
+    out = [S.BaseFieldVec.uninitialized(1 << m) for _ in range(n_cols)]
+    S.lde_columns_async(cols, cols, out, [log_n] * n_cols, blowup, tw, itw, 1 << coset.log_size)
+    S.synchronize()
+    otw, oitw = O.precompute_twiddles(coset.initial_index, coset.step_size, coset.log_size)
+    ocoef, olde = O.lde_columns([host[c] for c in sorted(host)], blowup, otw, oitw)
+    for i, c in enumerate(sorted(host)):
+        assert (cols[c].to_numpy() == ocoef[i]).all(), c
+        assert (out[c].to_numpy() == olde[i]).all(), c
