@@ -47,8 +47,12 @@ void qm31_powers_async(const qm31* d_alpha, uint32_t n, uint32_t* d_powers, uint
 void wide_fib_quotients_async(uint32_t* const q[4], const uint32_t* const* d_trace, const uint32_t* powers,
                               const uint32_t* dinv, uint32_t n_rows, uint32_t n_cols, uint32_t n_jobs, uint64_t js);
 size_t eval_at_point_columns_scratch_bytes(uint32_t n_cols, uint32_t L);
-void eval_at_point_columns_async(const uint32_t* const* d_cols, uint32_t n_cols, uint32_t L, const qm31* d_point,
-                                 qm31* d_out, void* d_scratch, uint32_t n_jobs, uint64_t js);
+namespace eap {
+struct Factors;
+}
+void eval_at_points_columns_async(const uint32_t* const* d_cols, uint32_t n_cols, uint32_t L, uint32_t n_points,
+                                  const qm31* d_points, const eap::Factors* d_factors, qm31* d_out, void* d_scratch,
+                                  uint32_t n_jobs, uint64_t js);
 size_t quotient_single_point_scratch_bytes(uint32_t n_cols, uint32_t max_log);
 void accumulate_quotients_single_point_async(uint32_t hi, uint32_t hs, uint32_t log_size,
                                              const uint32_t* const* d_cols, uint32_t n_cols, const qm31* d_point,
@@ -617,8 +621,8 @@ void Job::enqueue(const uint64_t* seeds) {
       timed("channel_oods_point", [&] { k_mix_root_draw_point<<<one, 1, 0, stream>>>(jb, layers_q[0], js); });
   }
 
-  eval_at_point_columns_async(t_coeffs, C, ln, jb->z, samples, eap_scratch, K, js);
-  eval_at_point_columns_async(t_comp, 4, ln + 1, jb->z, samples + C, eap_scratch, K, js);
+  eval_at_points_columns_async(t_coeffs, C, ln, 1, jb->z, nullptr, samples, eap_scratch, K, js);
+  eval_at_points_columns_async(t_comp, 4, ln + 1, 1, jb->z, nullptr, samples + C, eap_scratch, K, js);
   timed("channel_samples", [&] { k_mix_samples_draw<<<one, TREE_NT, 0, stream>>>(jb, samples, C + 4, js); });
 
   uint32_t* f1c[4] = {f1, f1 + cs(2 * n), f1 + 2 * cs(2 * n), f1 + 3 * cs(2 * n)};

@@ -183,8 +183,9 @@ void Pool::release_cached() {
 static Staging& take_staging(size_t bytes) {
   Context& c = g_ctx;
   for (auto& st : c.staging) {
+    if (st.held || st.cap < bytes) continue;
     if (st.busy && hipEventQuery(st.done) == hipSuccess) st.busy = false;
-    if (!st.busy && st.cap >= bytes) return st;
+    if (!st.busy) return st;
   }
   Staging st{};
   st.cap = std::max<size_t>(bytes, 64 << 10);
@@ -232,6 +233,19 @@ void upload_to(void* dev, const void* host, size_t bytes) {
   }
   hip_check(hipEventRecord(st.done, g_ctx.cur), "hipEventRecord");
   st.busy = true;
+}
+
+HostResult::HostResult(size_t bytes) {
+  Staging& st = take_staging(bytes);
+  index_ = &st - g_ctx.staging.data();
+  st.busy = true;
+  st.held = true;  // taken until the destructor, whose event marks the last kernel that writes to it
+  p_ = st.host;
+}
+HostResult::~HostResult() {
+  Staging& st = g_ctx.staging[index_];
+  (void)hipEventRecord(st.done, g_ctx.cur);
+  st.held = false;
 }
 
 DevBuf upload(const void* host, size_t bytes) {

@@ -72,6 +72,7 @@ struct Staging {
   size_t cap;
   hipEvent_t done;
   bool busy;
+  bool held;  // by a HostResult
 };
 
 struct TimedLaunch {
@@ -140,6 +141,26 @@ struct DevBuf {
 DevBuf upload(const void* host, size_t bytes);
 // Same into existing device memory.
 void upload_to(void* dev, const void* host, size_t bytes);
+
+// Pinned host memory that a kernel on ctx().cur writes small results to: read it after
+// synchronising that stream.  (A device buffer and a copy to pageable memory cost a copy kernel
+// and the runtime's own staging, about 15 us behind the last kernel.)
+constexpr size_t HOST_RESULT_MAX = 1 << 20;
+class HostResult {
+ public:
+  explicit HostResult(size_t bytes);
+  ~HostResult();
+  HostResult(const HostResult&) = delete;
+  HostResult& operator=(const HostResult&) = delete;
+  template <class T>
+  T* as() const {
+    return static_cast<T*>(p_);
+  }
+
+ private:
+  size_t index_;
+  void* p_;
+};
 
 // Launch bookkeeping: when kernel timing is on, bracket the launch with events.
 void launch_begin(const char* name);

@@ -82,3 +82,20 @@ def test_extension_on_matrix_cores(log_n, n_cols, blowup):
     for i, c in enumerate(sorted(host)):
         assert (cols[c].to_numpy() == ocoef[i]).all(), c
         assert (out[c].to_numpy() == olde[i]).all(), c
+
+
+@pytest.mark.parametrize("log_n,n_cols,n_points", [(11, 3, 2), (12, 1, 1), (12, 33, 3), (13, 5, 2), (14, 700, 1),
+                                                   (15, 3, 5), (17, 2, 2), (18, 9, 2), (20, 1, 3), (23, 1, 2)])
+def test_oods_values(log_n, n_cols, n_points):
+    """Batched evaluation at points: one block per column up to the shapes with several ranges per
+    column and one, two or more points (the last of an odd number alone); both entry points."""
+    rng = np.random.default_rng(log_n * 100 + n_cols)
+    host = rng.integers(0, S.P, (n_cols, 1 << log_n), dtype=np.uint32)
+    host[0][:] = S.P - 1
+    cols = [S.BaseFieldVec.from_numpy(h) for h in host]
+    pts = [S.random_circle_point_qm31(rng) for _ in range(n_points)]
+    got = S.eval_at_points_columns(cols, pts)
+    assert got == S.eval_at_points_columns(cols, pts, noalloc=True)
+    for c in {0, n_cols // 2, n_cols - 1}:
+        for k in range(n_points):
+            assert got[k][c] == tuple(int(v) for v in O.eval_at_point(host[c], *pts[k])), (c, k)
