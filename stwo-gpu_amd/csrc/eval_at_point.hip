@@ -168,19 +168,7 @@ __global__ __launch_bounds__(256) void basis_tables_kernel(const Factors* __rest
     const uint32_t c[4] = {v.x.a, v.x.b, v.y.a, v.y.b};
     // matrix operand of 8 values of r: lane row + 32 (bit 2 of r), word r mod 4
     uint32_t* const q = jptr(mid, jo) + 4 * (64 * (t >> 3) + 32 * ((t >> 2) & 1)) + (t & 3);
-#pragma unroll
-    for (uint32_t k = 0; k < 4; k++) {
-      uint32_t w[4];
-#pragma unroll
-      for (uint32_t j = 0; j < 4; j++) w[j] = mm::limbs(mm::rot31(c[k], 8 * j));
-#pragma unroll
-      for (uint32_t i = 0; i < 4; i++) {
-        uint32_t b = 0;
-#pragma unroll
-        for (uint32_t j = 0; j < 4; j++) b |= ((w[j] >> (8 * i)) & 0xff) << (8 * j);
-        q[4 * (4 * (4 * p + k) + i)] = b;
-      }
-    }
+    mm::operand_rows(c, q + 16 * 4 * p);
     return;
   }
   t -= n_mid;
@@ -189,14 +177,6 @@ __global__ __launch_bounds__(256) void basis_tables_kernel(const Factors* __rest
     jptr(lo, jo)[p * n_lo + t] = product(t, 0, LO_BITS);
   else if (t - n_lo < n_hi)
     jptr(hi, jo)[p * n_hi + t - n_lo] = product(t - n_lo, LO_BITS + r_log, L - LO_BITS - r_log);
-}
-
-// limb sums over up to 256 values of r (|sum| <= 2^24) to the canonical value: exact in 64 bits,
-// made nonnegative by 2^18 P
-__device__ __forceinline__ uint32_t join64(int a0, int a1, int a2, int a3) {
-  const int64_t v = ((((((int64_t)a3 << 8) + a2) << 8) + a1) << 8) + a0;
-  const uint64_t u = (uint64_t)(v + ((int64_t)P << 18));  // < 2^50
-  return canon((uint32_t)(u & P) + (uint32_t)(u >> 31));
 }
 
 template <int W>
@@ -260,7 +240,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void g
     uint32_t v[4];
 #pragma unroll
     for (int q = 0; q < 4; q++)
-      v[q] = join64(acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]);
+      v[q] = mm::join64(acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]);
     const uint32_t z0 = (uint32_t)__shfl_xor((int)(g ? v[0] : v[2]), 32);
     const uint32_t z1 = (uint32_t)__shfl_xor((int)(g ? v[1] : v[3]), 32);
     const qm31 val = g ? qm31{{z0, v[2]}, {z1, v[3]}} : qm31{{v[0], z0}, {v[1], z1}};
@@ -481,11 +461,11 @@ extern "C" int stwo_hip_eval_at_points_columns(const uint32_t* const* columns, u
     }
     memcpy(host.data() + p_bytes, columns, (size_t)n_cols * sizeof(void*));
     // input and scratch in one block; the last kernel writes the values to host memory (more than
-    // HOST_RESULT_MAX bytes of them to the device first, which keeps the pinned buffers small)
+    // HOST_BLOCK_MAX bytes of them to the device first, which keeps the pinned buffers small)
     const size_t in_bytes = (host.size() + 255) & ~(size_t)255;
     const size_t out_bytes = sizeof(qm31) * n_cols * (size_t)n_points;
     const size_t scratch_bytes = (eval_at_point_columns_scratch_bytes(n_cols, log_size) + 255) & ~(size_t)255;
-    const bool to_host = out_bytes <= HOST_RESULT_MAX;
+    const bool to_host = out_bytes <= HOST_BLOCK_MAX;
     DevBuf dev(in_bytes + scratch_bytes + (to_host ? 0 : out_bytes));
     unsigned char* const base = dev.as<unsigned char>();
     upload_to(base, host.data(), host.size());
@@ -495,7 +475,7 @@ extern "C" int stwo_hip_eval_at_points_columns(const uint32_t* const* columns, u
                                    gemv ? dev.as<eap::Factors>() : nullptr, out, base + in_bytes, 1, 0);
     };
     if (to_host) {
-      HostResult out(out_bytes);
+      HostBlock out(out_bytes);
       enqueue(out.as<qm31>());
       sync();
       memcpy(values, out.as<void>(), out_bytes);

@@ -199,13 +199,6 @@ constexpr int CT = 512;
 __host__ __device__ constexpr uint32_t lds_pos(uint32_t q) { return q + ((q >> 4) << 2); }
 constexpr uint32_t lds_words(uint32_t values) { return values / 16 * 20; }
 
-// Blocks go round-robin to the 8 XCDs, each with its own L2; block b takes place
-// (b mod 8) G / 8 + b / 8 of the order, so an XCD's blocks are neighbours in it.
-__device__ __forceinline__ uint32_t xcd_order() {
-  const uint32_t G = gridDim.x, q = G / 8, rem = G % 8, x = blockIdx.x % 8;
-  return x * q + min(x, rem) + blockIdx.x / 8;
-}
-
 // NS (forward): source slots of stage C that hold coefficients, 8 / 2^blowup; the rest are zero.
 // NT: streaming accesses.
 template <bool INV, int K, int NS, bool NT>

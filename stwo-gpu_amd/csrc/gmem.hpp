@@ -68,15 +68,16 @@ struct BufCol {
   static __device__ __forceinline__ __amdgpu_buffer_rsrc_t make(const void* p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(uniform(p)), (short)0, -1, 0x00020000);
   }
-  // word i + s (i per lane, s uniform)
+  // word i + s (i per lane, s uniform).  NT: a streaming access (nontemporal hint), for buffers
+  // larger than the caches that pass through once
+  template <bool NT = false>
   __device__ __forceinline__ uint32_t load(uint32_t i, uint32_t s) const {
-    return __builtin_amdgcn_raw_buffer_load_b32(rs, i * 4u, s * 4u, 0);
+    return __builtin_amdgcn_raw_buffer_load_b32(rs, i * 4u, s * 4u, NT ? 2 : 0);
   }
   __device__ __forceinline__ void store(uint32_t v, uint32_t i, uint32_t s) const {
     __builtin_amdgcn_raw_buffer_store_b32(v, rs, i * 4u, s * 4u, 0);
   }
-  // words i + s .. i + s + 3.  NT: a streaming access (nontemporal hint), for buffers larger than
-  // the caches that pass through once
+  // words i + s .. i + s + 3
   template <bool NT = false>
   __device__ __forceinline__ uint4 load4(uint32_t i, uint32_t s) const {
     const auto v = __builtin_amdgcn_raw_buffer_load_b128(rs, i * 4u, s * 4u, NT ? 2 : 0);
@@ -99,5 +100,12 @@ struct BufCol {
     __builtin_amdgcn_raw_buffer_store_b64(u32x2{v0, v1}, rs, i * 4u, s * 4u, NT ? 2 : 0);
   }
 };
+
+// Blocks go round-robin to the 8 XCDs, each with its own L2; block b takes place
+// (b mod 8) G / 8 + b / 8 of the order, so an XCD's blocks are neighbours in it.
+__device__ __forceinline__ uint32_t xcd_order() {
+  const uint32_t G = gridDim.x, q = G / 8, rem = G % 8, x = blockIdx.x % 8;
+  return x * q + min(x, rem) + blockIdx.x / 8;
+}
 
 }  // namespace sh

@@ -88,6 +88,31 @@ __host__ __device__ __forceinline__ uint32_t join(uint32_t a0, uint32_t a1, uint
   }
 }
 
+// The limb rows of four entries c[0..3] of a matrix operand: row 4 k + i of the rows from q on
+// (16 bytes apart) gets, in its word, limb i of c[k] 2^(8j) for the digits j.
+__host__ __device__ __forceinline__ void operand_rows(const uint32_t (&c)[4], uint32_t* q) {
+#pragma unroll
+  for (uint32_t k = 0; k < 4; k++) {
+    uint32_t w[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; j++) w[j] = limbs(rot31(c[k], 8 * j));
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+      uint32_t b = 0;
+#pragma unroll
+      for (uint32_t j = 0; j < 4; j++) b |= ((w[j] >> (8 * i)) & 0xff) << (8 * j);
+      q[4 * (4 * k + i)] = b;
+    }
+  }
+}
+// limb sums of many products (each |sum| <= 2^29: up to 2^13 terms of 4 digits) to the canonical
+// value: exact in 64 bits, made nonnegative by 2^23 P
+__host__ __device__ __forceinline__ uint32_t join64(int a0, int a1, int a2, int a3) {
+  const int64_t v = ((((((int64_t)a3 << 8) + a2) << 8) + a1) << 8) + a0;
+  const uint64_t u = (uint64_t)(v + ((int64_t)P << 23));  // < 2^55
+  return canon((uint32_t)(u & P) + (uint32_t)(u >> 31));
+}
+
 struct Mat {
   v4i c[4];  // chunks (T, s) at 2T + s
 };

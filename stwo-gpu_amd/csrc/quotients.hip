@@ -12,15 +12,17 @@
 //
 // MI355X design: the per-batch sums of a_j and b_j and the factor c (shared by
 // every sample of a batch, since c depends only on P) are folded on the host, so
-// a row costs one QM31 x M31 multiply-accumulate per sample, done on 64-bit
-// lazy sums (v_mad_u64_u32) and reduced once per batch.  Sample tables are
-// uniform across the wavefront and are read with scalar loads.
+// what is left per row is sum_j alpha_j col_j[row] per batch: for up to 4 batches
+// a contraction over the columns on the matrix cores (accumulate_mm_kernel; for few samples
+// accumulate_cols_kernel), beyond that multiply-accumulates on 64-bit lazy sums, batch by
+// batch (accumulate_kernel).
 #include <cstring>
 #include <map>
 #include <vector>
 
 #include "field.hpp"
 #include "gmem.hpp"
+#include "mfma_m31.hpp"
 #include "runtime.hpp"
 
 namespace sh {
@@ -120,14 +122,44 @@ __global__ __launch_bounds__(256) void accumulate_kernel(DomainTables T, uint32_
   o3[row] = acc.y.b;
 }
 
-// Column-major form for up to 4 batches: each sampled column value of a row is loaded
-// once and multiplied into the sums of all NB batches, with alpha = 0 for a batch that
-// does not sample the column.  Per column the host provides NB alphas (one uniform
-// 16 * NB-byte record), so the loop has no data-dependent branches; loads run one group
-// of QG columns ahead of the arithmetic.  A batch's sums are folded after every fourth
-// product taken into them: a product of two values below P is at most (P - 1)^2 =
-// 2^62 - 2^33 + 1, and a folded sum is below 2^34, so four products on top of it stay
-// below 2^64.
+__device__ __forceinline__ cm31 batch_denominator(const Batch& B, pt p) {
+  return csub(cmul(cm31{sub(B.prx.a, p.x), B.prx.b}, B.piy), cmul(cm31{sub(B.pry.a, p.y), B.pry.b}, B.pix));
+}
+
+// the accumulation over the batches at p, from each batch's sum: one CM31 inversion for the NB
+// denominators (prefix products, Montgomery's trick)
+template <int NB>
+__device__ __forceinline__ qm31 combine(const Batch* __restrict__ batches, const qm31* sum, pt p) {
+  cm31 d[NB], pre[NB];
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    d[b] = batch_denominator(batches[b], p);
+    pre[b] = b == 0 ? d[0] : cmul(pre[b - 1], d[b]);
+  }
+  cm31 inv_all = cinv(pre[NB - 1]);
+  cm31 dinv[NB];
+#pragma unroll
+  for (int b = NB - 1; b > 0; b--) {
+    dinv[b] = cmul(inv_all, pre[b - 1]);
+    inv_all = cmul(inv_all, d[b]);
+  }
+  dinv[0] = inv_all;
+  qm31 r = qzero();
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    const Batch& B = batches[b];
+    const qm31 num = qsub(qmul(B.c, sum[b]), qadd(qscale(B.a_sum, p.y), B.b_sum));
+    r = qadd(qmul(r, B.coeff), qmul_cm(num, dinv[b]));
+  }
+  return r;
+}
+
+// Column-major form for up to 4 batches and few samples (or more columns than MM_MAX_SLOTS): each
+// sampled column value of a row is loaded once and multiplied into the sums of all NB batches,
+// with alpha = 0 for a batch that does not sample the column; loads run one group of QG columns
+// ahead of the arithmetic.  A batch's sums are folded after every fourth product taken into
+// them: a product of two values below P is at most (P - 1)^2 = 2^62 - 2^33 + 1, and a folded
+// sum is below 2^34, so four products on top of it stay below 2^64.
 template <int NB>
 struct ColSlot {
   const uint32_t* col;  // the column (device pointer)
@@ -136,35 +168,16 @@ struct ColSlot {
   qm31 alpha[NB];
 };
 
-__device__ __forceinline__ cm31 batch_denominator(const Batch& B, pt p) {
-  return csub(cmul(cm31{sub(B.prx.a, p.x), B.prx.b}, B.piy), cmul(cm31{sub(B.pry.a, p.y), B.pry.b}, B.pix));
-}
-__device__ __forceinline__ qm31 finish_batch(const Batch& B, const uint64_t (&s)[4], pt p, cm31 dinv, qm31 acc) {
-  qm31 sum = {{reduce63(s[0]), reduce63(s[1])}, {reduce63(s[2]), reduce63(s[3])}};
-  qm31 num = qsub(qmul(B.c, sum), qadd(qscale(B.a_sum, p.y), B.b_sum));
-  return qadd(qmul(acc, B.coeff), qmul_cm(num, dinv));
-}
-
 constexpr int QG = 16;  // columns per load group (a multiple of the fold period 4; 8: 6 % slower at 200 x 2^21)
 
-// js: byte stride between the jobs of a batched launch (blockIdx.z = job): the slot and batch
-// tables and the outputs move by the job's offset (the slots already hold that job's columns)
 template <int NB>
 __global__ __launch_bounds__(256) void accumulate_cols_kernel(DomainTables T, uint32_t log_size,
                                                               const ColSlot<NB>* __restrict__ slots,
                                                               uint32_t n_slots, const Batch* __restrict__ batches,
                                                               uint32_t* __restrict__ o0, uint32_t* __restrict__ o1,
-                                                              uint32_t* __restrict__ o2, uint32_t* __restrict__ o3,
-                                                              uint64_t js) {
+                                                              uint32_t* __restrict__ o2, uint32_t* __restrict__ o3) {
   uint32_t row = blockIdx.x * blockDim.x + threadIdx.x;
   if (row >= (1u << log_size)) return;
-  const uint64_t jo = job_offset(js);
-  slots = jptr(slots, jo);
-  batches = jptr(batches, jo);
-  o0 = jptr(o0, jo);
-  o1 = jptr(o1, jo);
-  o2 = jptr(o2, jo);
-  o3 = jptr(o3, jo);
   uint64_t s[NB][4];
 #pragma unroll
   for (int b = 0; b < NB; b++) s[b][0] = s[b][1] = s[b][2] = s[b][3] = 0;
@@ -206,28 +219,211 @@ __global__ __launch_bounds__(256) void accumulate_cols_kernel(DomainTables T, ui
     for (int i = 0; i < QG; i++) v[i] = vn[i];
   }
   const pt p = domain_point(T, brev(row, log_size));
-  // one CM31 inversion for the NB denominators (prefix products, Montgomery's trick)
-  cm31 d[NB], pre[NB];
+  qm31 sum[NB];
 #pragma unroll
-  for (int b = 0; b < NB; b++) {
-    d[b] = batch_denominator(batches[b], p);
-    pre[b] = b == 0 ? d[0] : cmul(pre[b - 1], d[b]);
-  }
-  cm31 inv_all = cinv(pre[NB - 1]);
-  cm31 dinv[NB];
-#pragma unroll
-  for (int b = NB - 1; b > 0; b--) {
-    dinv[b] = cmul(inv_all, pre[b - 1]);
-    inv_all = cmul(inv_all, d[b]);
-  }
-  dinv[0] = inv_all;
-  qm31 acc = qzero();
-#pragma unroll
-  for (int b = 0; b < NB; b++) acc = finish_batch(batches[b], s[b], p, dinv[b], acc);
+  for (int b = 0; b < NB; b++)
+    sum[b] = {{reduce63(s[b][0]), reduce63(s[b][1])}, {reduce63(s[b][2]), reduce63(s[b][3])}};
+  const qm31 acc = combine<NB>(batches, sum, p);
   o0[row] = acc.x.a;
   o1[row] = acc.x.b;
   o2[row] = acc.y.a;
   o3[row] = acc.y.b;
+}
+
+// Column-major form for up to 4 batches, on the matrix cores: the sums sum_j alpha_j col_j[row] of
+// all batches are one contraction over the columns.  v_mfma_i32_32x32x32_i8 on signed byte digits
+// (mfma_m31.hpp) takes a step of 8 columns (4 digits each) of 32 rows times 8 outputs of 4 limbs,
+// two batches to an instruction; a column that a batch does not sample has weight 0 there.  Two
+// and a half VALU instructions per value instead of four 64-bit multiply-adds per sample and their
+// folds leave the kernel bound by the column reads.
+//
+// The reads need about 64 KB per CU on their way.  Held in registers they cost the occupancy, and
+// the compiler waits for all of them at each turn of the loop (360 us at 200 columns of 2^21, 3
+// points).  So they go straight to LDS: a wave's 64 rows of DEPTH steps of columns are a ring that
+// only this wave reads, after a wait that leaves the newer steps in flight; no registers, no
+// barrier.  The operand tiles are the block's, loaded the same way CHUNK steps at a time into the
+// half that is not being read (one barrier a chunk; read from L2 by every wave they would be as
+// many bytes as the columns).  The LDS reads and their wait are one asm statement: reads through
+// the compiler would again wait for every load.  200 columns of 2^21, 3 points: 373 -> 320 us per
+// call, the kernel 300 (5.7 TB/s); a ring of 4 steps is no faster; blocks in XCD order 598 us
+// instead of 624 at 200 columns of 2^22 (columns not padded apart share an XCD's lines).
+constexpr uint32_t KSTEP = 8;            // columns per step
+constexpr uint32_t MM_MAX_SLOTS = 8192;  // columns: join64's bound on the limb sums
+constexpr uint32_t MM_WAVES = 8;         // per block; 64 rows each
+constexpr uint32_t DEPTH = 3;            // steps of columns on their way into a wave's ring
+constexpr uint32_t RING = DEPTH * KSTEP * 64, TILE = 256;  // words of a ring, of an operand tile
+// Values from which the column reads are nontemporal (more than the caches hold: 200 columns of
+// 2^22, 1 point: 597 us instead of 634; below, 64 columns of 2^20: 84 us plain, 90 nontemporal).
+constexpr uint64_t MM_STREAM = 1ull << 27;
+// Samples from which the matrix form is taken, for one batch and for more.  Its weights are
+// expanded by a launch of their own instead of copied (3 us), and a batch alone fills half an
+// operand tile.  One point, cols / matrix: 96 columns of 2^20 93 / 102 us, 128 columns 120 / 112,
+// 64 of 2^12 18.7 / 21.9, 256 of 2^12 38 / 34.  Two to four points: 8 columns of 2^12, 2 points
+// 17.9 / 20.1 us, 32 columns 24.5 / 21.7; 32 columns of 2^20, 2 points 82 / 56.
+constexpr uint32_t FEW_ONE = 128, FEW = 32;
+constexpr uint32_t mm_tiles(uint32_t n_batches) { return (n_batches + 1) / 2; }
+constexpr uint32_t padded_slots(uint32_t n_cols) { return (n_cols + KSTEP - 1) / KSTEP * KSTEP; }
+
+// word of the weights of slot, batch: the first of its 16 rows (4 words apart)
+__host__ __device__ __forceinline__ uint32_t weight_word(uint32_t slot, uint32_t batch, uint32_t tiles) {
+  return ((slot / KSTEP * tiles + batch / 2) * 64 + ((slot >> 2) & 1) * 32 + (batch & 1) * 16) * 4 + (slot & 3);
+}
+
+// From a host image (pinned memory or an upload) to the kernel's tables: column pointers and
+// batches copied, alphas ([slot][batch], n_slots x n_batches) expanded to weights.
+__global__ __launch_bounds__(256) void weights_kernel(const uint2* __restrict__ ptrs, const qm31* __restrict__ alphas,
+                                                      const uint32_t* __restrict__ batch_words, uint32_t n_slots,
+                                                      uint32_t n_batches, uint2* d_ptrs, uint32_t* weights,
+                                                      uint32_t* d_batches) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t tiles = mm_tiles(n_batches);
+  if (t < n_slots) d_ptrs[t] = ptrs[t];
+  if (t < n_batches * (sizeof(Batch) / 4)) d_batches[t] = batch_words[t];
+  const uint32_t slot = t / (2 * tiles), b = t % (2 * tiles);
+  if (slot >= n_slots) return;
+  const qm31 v = b < n_batches ? alphas[slot * n_batches + b] : qzero();
+  const uint32_t c[4] = {v.x.a, v.x.b, v.y.a, v.y.b};
+  mm::operand_rows(c, weights + weight_word(slot, b, tiles));
+}
+
+// js: byte stride between the jobs of a batched launch (blockIdx.z = job): the tables and the
+// outputs move by the job's offset (the pointers already are that job's columns)
+template <int NB, bool NT>
+__global__ __launch_bounds__(MM_WAVES * 64) __attribute__((amdgpu_waves_per_eu(4))) void accumulate_mm_kernel(
+    DomainTables T, uint32_t log_size, const uint32_t* const* __restrict__ cols, const uint32_t* __restrict__ weights,
+    uint32_t n_steps, const Batch* __restrict__ batches, uint32_t* __restrict__ o0, uint32_t* __restrict__ o1,
+    uint32_t* __restrict__ o2, uint32_t* __restrict__ o3, uint64_t js) {
+  constexpr int MT = (int)mm_tiles(NB);
+  constexpr uint32_t CHUNK = MM_WAVES / MT;  // steps whose operand tiles the block loads together, a tile per wave
+  static_assert(CHUNK >= DEPTH, "a chunk's tiles are older than its first step's columns");
+  __shared__ __align__(16) uint32_t lds[MM_WAVES * RING + 2 * MM_WAVES * TILE];
+  (void)lds;
+  const uint64_t jo = job_offset(js);
+  cols = jptr(cols, jo);
+  batches = jptr(batches, jo);
+  uint32_t* const out[4] = {jptr(o0, jo), jptr(o1, jo), jptr(o2, jo), jptr(o3, jo)};
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t n_rows = 1u << log_size, place = (MM_WAVES * xcd_order() + wave) * 64;
+  // a wave past the domain's end repeats its first rows, a lane past it the last one
+  const uint32_t row0 = place < n_rows ? place : 0, row = min(lane, n_rows - 1 - row0);
+
+  mm::v16i acc[MT][2] = {};  // [tile][rows of the wave's lower or upper 32 lanes]
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef __attribute__((address_space(3))) uint32_t lds_word;
+  lds_word* const ring = (lds_word*)lds + wave * RING;
+  lds_word* const wring = (lds_word*)lds + MM_WAVES * RING;
+  constexpr int AUX = NT ? 2 : 0;
+  auto fetch = [&](const uint32_t* const (&p)[KSTEP], uint32_t slot) {
+#pragma unroll
+    for (uint32_t c = 0; c < KSTEP; c++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(BufCol(p[c] + row0).rs, ring + (slot * KSTEP + c) * 64, 4, row * 4, 0,
+                                               0, AUX);
+  };
+  auto pointers = [&](const uint32_t* (&p)[KSTEP], uint32_t step) {
+#pragma unroll
+    for (uint32_t c = 0; c < KSTEP; c++) p[c] = ld_uniform(cols, KSTEP * step + c);
+  };
+  const BufCol wbuf(jptr(weights, jo));
+  auto fetch_weights = [&](uint32_t chunk) {
+    const uint32_t tile = chunk * MM_WAVES + wave;
+    if (tile < n_steps * MT)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wbuf.rs, wring + ((chunk & 1) * MM_WAVES + wave) * TILE, 16, lane * 16,
+                                               tile * (4 * TILE), 0, 0);
+  };
+  fetch_weights(0);
+  for (uint32_t s = 0; s < DEPTH && s < n_steps; s++) {
+    const uint32_t* p[KSTEP];
+    pointers(p, s);
+    fetch(p, s);
+  }
+  const uint32_t x_lane = (uint32_t)(size_t)ring + (lane >> 5) * 1024 + (lane & 31) * 4;
+  const uint32_t w_lane = (uint32_t)(size_t)wring + lane * 16;
+  uint32_t slot = 0;
+  for (uint32_t s = 0; s < n_steps; s++) {
+    const uint32_t* p[KSTEP];
+    pointers(p, min(s + DEPTH, n_steps - 1));
+    // the loads come back in order: all but the newest DEPTH - 1 steps are there
+    if (s + DEPTH <= n_steps)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"i"((DEPTH - 1) * KSTEP) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (s % CHUNK == 0) {
+      // every wave's tile of this chunk is there (older than the step just waited for), and nobody
+      // reads the other half any more
+      __builtin_amdgcn_s_barrier();
+      fetch_weights(s / CHUNK + 1);
+    }
+    typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+    v2u x[4];
+    mm::v4i w[2];
+    const uint32_t xa = x_lane + slot * (KSTEP * 256), xb = xa + 128;
+    const uint32_t wa = w_lane + s % (2 * CHUNK) * (MT * 4 * TILE);
+    if constexpr (MT == 2) {
+      asm volatile(
+          "ds_read2st64_b32 %0, %6 offset0:0 offset1:1\n"
+          "ds_read2st64_b32 %1, %6 offset0:2 offset1:3\n"
+          "ds_read_b128 %4, %8\n"
+          "ds_read_b128 %5, %8 offset:1024\n"
+          "ds_read2st64_b32 %2, %7 offset0:0 offset1:1\n"
+          "ds_read2st64_b32 %3, %7 offset0:2 offset1:3\n"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(w[0]), "=&v"(w[1])
+          : "v"(xa), "v"(xb), "v"(wa)
+          : "memory");
+    } else {
+      asm volatile(
+          "ds_read2st64_b32 %0, %5 offset0:0 offset1:1\n"
+          "ds_read2st64_b32 %1, %5 offset0:2 offset1:3\n"
+          "ds_read_b128 %4, %7\n"
+          "ds_read2st64_b32 %2, %6 offset0:0 offset1:1\n"
+          "ds_read2st64_b32 %3, %6 offset0:2 offset1:3\n"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(w[0])
+          : "v"(xa), "v"(xb), "v"(wa)
+          : "memory");
+    }
+    if (s + DEPTH < n_steps) fetch(p, slot);  // into the slot that was just read
+    slot = slot + 1 == DEPTH ? 0 : slot + 1;
+    mm::v4i lo, hi;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      lo[i] = (int)mm::digits(x[i / 2][i & 1]);
+      hi[i] = (int)mm::digits(x[2 + i / 2][i & 1]);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+      acc[t][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[t], lo, acc[t][0], 0, 0, 0);
+      acc[t][1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(w[t], hi, acc[t][1], 0, 0, 0);
+    }
+  }
+#endif
+  // registers 4q .. 4q + 3 hold the limbs of output 2q + (lane / 32) of either half's rows: the
+  // swap gives each lane its own row's outputs 2q and 2q + 1
+  qm31 sum[2 * MT];
+#pragma unroll
+  for (int t = 0; t < MT; t++) {
+    uint32_t e[4], o[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const mm::v16i &a = acc[t][0], &b = acc[t][1];
+      e[q] = mm::join64(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
+      o[q] = mm::join64(b[4 * q], b[4 * q + 1], b[4 * q + 2], b[4 * q + 3]);
+#if defined(__HIP_DEVICE_COMPILE__)
+      const auto z = __builtin_amdgcn_permlane32_swap(e[q], o[q], false, false);
+      e[q] = z[0];
+      o[q] = z[1];
+#endif
+    }
+    sum[2 * t] = {{e[0], o[0]}, {e[1], o[1]}};
+    sum[2 * t + 1] = {{e[2], o[2]}, {e[3], o[3]}};
+  }
+  if (lane >= n_rows - row0 || place >= n_rows) return;
+  const pt p = domain_point(T, brev(row0 + row, log_size));
+  const qm31 r = combine<NB>(batches, sum, p);
+  const uint32_t res[4] = {r.x.a, r.x.b, r.y.a, r.y.b};
+#pragma unroll
+  for (int k = 0; k < 4; k++) BufCol(out[k] + row0).store(res[k], row, 0);
 }
 
 // One batch (every column sampled once at one point) built on the device from a
@@ -237,29 +433,36 @@ constexpr uint32_t SB_NT = 256;
 __global__ __launch_bounds__(SB_NT) void single_batch_kernel(const uint32_t* const* __restrict__ cols,
                                                              const qm31* __restrict__ point,
                                                              const qm31* __restrict__ values, uint32_t count,
-                                                             const qm31* __restrict__ rc_dev, ColSlot<1>* ss,
-                                                             uint32_t n_slots, Batch* bs, uint64_t js) {
+                                                             const qm31* __restrict__ rc_dev, const uint32_t** ptrs,
+                                                             uint32_t* weights, uint32_t n_slots, Batch* bs,
+                                                             uint64_t js) {
   __shared__ qm31 sa[SB_NT], sb[SB_NT];
   // batched jobs (blockIdx.z): the slots get the job's own column pointers
   const uint64_t jo = job_offset(js);
   point = jptr(point, jo);
   values = jptr(values, jo);
   rc_dev = jptr(rc_dev, jo);
-  ss = jptr(ss, jo);
+  ptrs = jptr(ptrs, jo);
+  weights = jptr(weights, jo);
   bs = jptr(bs, jo);
   const qm31 px = point[0], py = point[1], rc = *rc_dev;
   const qm31 c = qsub(qm31{py.x, cneg(py.y)}, py);
   qm31 la = qzero(), lb = qzero();
-  for (uint32_t j = threadIdx.x; j < count; j += SB_NT) {
-    const qm31 alpha = qpow(rc, j + 1);
-    const qm31 v = values[j];
-    const qm31 a = qsub(qm31{v.x, cneg(v.y)}, v);
-    const qm31 bb = qsub(qmul(v, c), qmul(a, py));
-    la = qadd(la, qmul(alpha, a));
-    lb = qadd(lb, qmul(alpha, bb));
-    ss[j] = ColSlot<1>{jptr(cols[j], jo), 1, 0, {alpha}};
+  for (uint32_t j = threadIdx.x; j < n_slots; j += SB_NT) {
+    ptrs[j] = jptr(cols[j < count ? j : 0], jo);
+    qm31 alpha = qzero();  // slots past the last column weigh nothing
+    if (j < count) {
+      alpha = qpow(rc, j + 1);
+      const qm31 v = values[j];
+      const qm31 a = qsub(qm31{v.x, cneg(v.y)}, v);
+      const qm31 bb = qsub(qmul(v, c), qmul(a, py));
+      la = qadd(la, qmul(alpha, a));
+      lb = qadd(lb, qmul(alpha, bb));
+    }
+    const uint32_t w[4] = {alpha.x.a, alpha.x.b, alpha.y.a, alpha.y.b}, none[4] = {0, 0, 0, 0};
+    mm::operand_rows(w, weights + weight_word(j, 0, 1));
+    mm::operand_rows(none, weights + weight_word(j, 1, 1));
   }
-  for (uint32_t j = count + threadIdx.x; j < n_slots; j += SB_NT) ss[j] = ColSlot<1>{jptr(cols[0], jo), 0, 0, {qzero()}};
   sa[threadIdx.x] = la;
   sb[threadIdx.x] = lb;
   __syncthreads();
@@ -286,17 +489,26 @@ __global__ __launch_bounds__(256) void zero_kernel(uint32_t n, uint32_t* o0, uin
 
 }  // namespace quot
 
-static uint32_t padded_slots(uint32_t n_cols) { return (n_cols + quot::QG - 1) / quot::QG * quot::QG; }
-// slots: the padded loop range plus QG trailing pad slots
-static size_t slot_bytes(uint32_t n_slots) {
-  return (sizeof(quot::ColSlot<1>) * (n_slots + quot::QG) + 255) & ~(size_t)255;
-}
-static constexpr size_t BATCH_BYTES = (sizeof(quot::Batch) + 255) & ~(size_t)255;
-// scratch of accumulate_quotients_single_point_async: slots | batch (the domain tables
-// come from the library's per-domain cache)
+// tables of an accumulate_mm launch: pointers | weights | batches
+namespace {
+struct MmLayout {
+  size_t weights, batches, end;
+  MmLayout(uint32_t n_slots, uint32_t n_batches) {
+    auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+    weights = up(sizeof(void*) * n_slots);
+    batches = weights + up((size_t)(n_slots / quot::KSTEP) * quot::mm_tiles(n_batches) * (4 * quot::TILE));
+    end = batches + up(sizeof(quot::Batch) * n_batches);
+  }
+};
+template <int NB>
+void launch_mm(uint32_t hi, uint32_t hs, uint32_t log_size, const void* tables, uint32_t n_slots, uint32_t* const out[4],
+               uint32_t n_jobs, uint64_t js);
+}  // namespace
+// scratch of accumulate_quotients_single_point_async (the domain tables come from the library's
+// per-domain cache)
 size_t quotient_single_point_scratch_bytes(uint32_t n_cols, uint32_t max_log) {
   (void)max_log;
-  return slot_bytes(padded_slots(std::max<uint32_t>(n_cols, 1))) + BATCH_BYTES;
+  return MmLayout(quot::padded_slots(std::max<uint32_t>(n_cols, 1)), 1).end;
 }
 
 // Fill the domain tables of CircleDomain(half coset (hi, hs), log log_size) at `dev`
@@ -340,25 +552,39 @@ void accumulate_quotients_single_point_async(uint32_t hi, uint32_t hs, uint32_t 
                                              const qm31* d_values, const qm31* d_rc, void* d_scratch,
                                              uint32_t* const out[4], uint32_t n_jobs, uint64_t js) {
   require(log_size >= 1 && log_size <= 30 && n_cols >= 1, "accumulate_quotients: bad sizes");
-  const uint32_t n_slots = padded_slots(n_cols);
-  quot::ColSlot<1>* ss = (quot::ColSlot<1>*)d_scratch;
-  quot::Batch* bs = (quot::Batch*)((char*)d_scratch + slot_bytes(n_slots));
-  const quot::DomainTables T = cached_domain_tables(hi, hs, log_size);
+  require(n_cols <= quot::MM_MAX_SLOTS, "accumulate_quotients: too many columns for one device-built batch");
+  const uint32_t n_slots = quot::padded_slots(n_cols);
+  const MmLayout Y(n_slots, 1);
+  char* const base = (char*)d_scratch;
   timed("quotient_constants", [&] {
-    quot::single_batch_kernel<<<dim3(1, 1, n_jobs), quot::SB_NT, 0, ctx().cur>>>(d_cols, d_point, d_values, n_cols,
-                                                                                d_rc, ss, n_slots + quot::QG, bs, js);
+    quot::single_batch_kernel<<<dim3(1, 1, n_jobs), quot::SB_NT, 0, ctx().cur>>>(
+        d_cols, d_point, d_values, n_cols, d_rc, (const uint32_t**)base, (uint32_t*)(base + Y.weights), n_slots,
+        (quot::Batch*)(base + Y.batches), js);
   });
-  timed("accumulate_quotients", [&] {
-    quot::accumulate_cols_kernel<1><<<dim3(ceil_div(1ull << log_size, 256), 1, n_jobs), 256, 0, ctx().cur>>>(
-        T, log_size, ss, n_slots, bs, out[0], out[1], out[2], out[3], js);
-  });
+  launch_mm<1>(hi, hs, log_size, base, n_slots, out, n_jobs, js);
 }
 
 namespace {
+template <int NB>
+void launch_mm(uint32_t hi, uint32_t hs, uint32_t log_size, const void* tables, uint32_t n_slots, uint32_t* const out[4],
+               uint32_t n_jobs, uint64_t js) {
+  const MmLayout Y(n_slots, NB);
+  const char* const base = (const char*)tables;
+  const quot::DomainTables T = cached_domain_tables(hi, hs, log_size);
+  constexpr uint32_t rows = quot::MM_WAVES * 64;  // per block
+  const auto kernel = (uint64_t)n_slots << log_size >= quot::MM_STREAM ? quot::accumulate_mm_kernel<NB, true>
+                                                                       : quot::accumulate_mm_kernel<NB, false>;
+  timed("accumulate_quotients", [&] {
+    kernel<<<dim3(ceil_div(1ull << log_size, rows), 1, n_jobs), quot::MM_WAVES * 64, 0, ctx().cur>>>(
+        T, log_size, (const uint32_t* const*)base, (const uint32_t*)(base + Y.weights), n_slots / quot::KSTEP,
+        (const quot::Batch*)(base + Y.batches), out[0], out[1], out[2], out[3], js);
+  });
+}
+
 // column-major launch: per sampled column one slot with the alpha of every batch (0 when
 // the batch does not sample it; a column sampled twice in one batch gets the sum)
 template <int NB>
-void launch_cols_nb(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols,
+void launch_slots(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols,
                     const std::vector<quot::Sample>& ss, const std::vector<quot::Batch>& bs, uint32_t* const out[4]) {
   std::map<uint32_t, quot::ColSlot<NB>> by_col;
   for (uint32_t b = 0; b < (uint32_t)NB; b++)
@@ -393,17 +619,69 @@ void launch_cols_nb(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t*
   const quot::DomainTables T = cached_domain_tables(hi, hs, log_size);
   timed("accumulate_quotients", [&] {
     quot::accumulate_cols_kernel<NB><<<ceil_div(1ull << log_size, 256), 256, 0, ctx().cur>>>(
-        T, log_size, dsl, n_loop, dbs, out[0], out[1], out[2], out[3], 0);
+        T, log_size, dsl, n_loop, dbs, out[0], out[1], out[2], out[3]);
   });
 }
-void launch_cols(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols,
+// column-major launch: per sampled column one slot with the alpha of every batch (0 when
+// the batch does not sample it; a column sampled twice in one batch gets the sum).  Returns
+// whether the columns are few enough for it.
+template <int NB>
+bool launch_matrix(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols, uint32_t n_cols,
+                    const std::vector<quot::Sample>& ss, const std::vector<quot::Batch>& bs, uint32_t* const out[4]) {
+  constexpr uint32_t NONE = ~0u;
+  std::vector<uint32_t> slot_of(n_cols, NONE);
+  uint32_t n_used = 0;
+  for (const quot::Sample& S : ss)
+    if (slot_of[S.col] == NONE) slot_of[S.col] = n_used++;
+  if (n_used > quot::MM_MAX_SLOTS) return false;
+  const uint32_t n_slots = quot::padded_slots(n_used);
+  // host image: pointers | alphas | batches
+  const size_t o_alpha = sizeof(void*) * n_slots, o_batch = o_alpha + sizeof(qm31) * NB * n_slots;
+  const size_t bytes = o_batch + sizeof(quot::Batch) * NB;
+  std::vector<unsigned char> big(bytes > HOST_BLOCK_MAX ? bytes : 0);
+  HostBlock pinned(big.empty() ? bytes : 16);
+  unsigned char* const host = big.empty() ? pinned.as<unsigned char>() : big.data();
+  memset(host, 0, bytes);
+  const uint32_t** ptrs = (const uint32_t**)host;
+  qm31* alphas = (qm31*)(host + o_alpha);
+  for (uint32_t b = 0; b < (uint32_t)NB; b++)
+    for (uint32_t j = 0; j < bs[b].count; j++) {
+      const quot::Sample& S = ss[bs[b].first + j];
+      const uint32_t slot = slot_of[S.col];
+      ptrs[slot] = h_cols[S.col];
+      alphas[slot * NB + b] = qadd(alphas[slot * NB + b], S.alpha);
+    }
+  for (uint32_t i = n_used; i < n_slots; i++) ptrs[i] = ptrs[0];
+  memcpy(host + o_batch, bs.data(), sizeof(quot::Batch) * NB);
+  const DevBuf up = big.empty() ? DevBuf() : upload(host, bytes);
+  const unsigned char* const src = big.empty() ? host : up.as<unsigned char>();
+  const MmLayout Y(n_slots, NB);
+  DevBuf d(Y.end);
+  char* const base = d.as<char>();
+  timed("quotient_constants", [&] {
+    const uint32_t threads = std::max<uint32_t>(n_slots * 2 * quot::mm_tiles(NB), NB * sizeof(quot::Batch) / 4);
+    quot::weights_kernel<<<ceil_div(threads, 256), 256, 0, ctx().cur>>>((const uint2*)src, (const qm31*)(src + o_alpha),
+                                                (const uint32_t*)(src + o_batch), n_slots, NB, (uint2*)base,
+                                                (uint32_t*)(base + Y.weights), (uint32_t*)(base + Y.batches));
+  });
+  launch_mm<NB>(hi, hs, log_size, base, n_slots, out, 1, 0);
+  return true;
+}
+template <int NB>
+void launch_cols_nb(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols, uint32_t n_cols,
+                    const std::vector<quot::Sample>& ss, const std::vector<quot::Batch>& bs, uint32_t* const out[4]) {
+  const bool few = ss.size() < (NB == 1 ? quot::FEW_ONE : quot::FEW);
+  if (few || !launch_matrix<NB>(hi, hs, log_size, h_cols, n_cols, ss, bs, out))
+    launch_slots<NB>(hi, hs, log_size, h_cols, ss, bs, out);
+}
+void launch_cols(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols, uint32_t n_cols,
                  const std::vector<quot::Sample>& ss, const std::vector<quot::Batch>& bs, uint32_t n_batches,
                  uint32_t* const out[4]) {
   switch (n_batches) {
-    case 1: launch_cols_nb<1>(hi, hs, log_size, h_cols, ss, bs, out); break;
-    case 2: launch_cols_nb<2>(hi, hs, log_size, h_cols, ss, bs, out); break;
-    case 3: launch_cols_nb<3>(hi, hs, log_size, h_cols, ss, bs, out); break;
-    default: launch_cols_nb<4>(hi, hs, log_size, h_cols, ss, bs, out);
+    case 1: launch_cols_nb<1>(hi, hs, log_size, h_cols, n_cols, ss, bs, out); break;
+    case 2: launch_cols_nb<2>(hi, hs, log_size, h_cols, n_cols, ss, bs, out); break;
+    case 3: launch_cols_nb<3>(hi, hs, log_size, h_cols, n_cols, ss, bs, out); break;
+    default: launch_cols_nb<4>(hi, hs, log_size, h_cols, n_cols, ss, bs, out);
   }
 }
 }  // namespace
@@ -463,7 +741,7 @@ void accumulate_quotients_async(uint32_t hi, uint32_t hs, uint32_t domain_size, 
     off += sizes[b];
   }
   if (n_batches >= 1 && n_batches <= 4) {
-    launch_cols(hi, hs, log_size, h_cols, ss, bs, n_batches, out);
+    launch_cols(hi, hs, log_size, h_cols, n_cols, ss, bs, n_batches, out);
     return;
   }
   if (ss.empty()) ss.push_back(quot::Sample{0, 0, qzero()});

@@ -235,14 +235,14 @@ void upload_to(void* dev, const void* host, size_t bytes) {
   st.busy = true;
 }
 
-HostResult::HostResult(size_t bytes) {
+HostBlock::HostBlock(size_t bytes) {
   Staging& st = take_staging(bytes);
   index_ = &st - g_ctx.staging.data();
   st.busy = true;
   st.held = true;  // taken until the destructor, whose event marks the last kernel that writes to it
   p_ = st.host;
 }
-HostResult::~HostResult() {
+HostBlock::~HostBlock() {
   Staging& st = g_ctx.staging[index_];
   (void)hipEventRecord(st.done, g_ctx.cur);
   st.held = false;

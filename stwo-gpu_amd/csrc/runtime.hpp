@@ -72,7 +72,7 @@ struct Staging {
   size_t cap;
   hipEvent_t done;
   bool busy;
-  bool held;  // by a HostResult
+  bool held;  // by a HostBlock
 };
 
 struct TimedLaunch {
@@ -142,16 +142,16 @@ DevBuf upload(const void* host, size_t bytes);
 // Same into existing device memory.
 void upload_to(void* dev, const void* host, size_t bytes);
 
-// Pinned host memory that a kernel on ctx().cur writes small results to: read it after
-// synchronising that stream.  (A device buffer and a copy to pageable memory cost a copy kernel
-// and the runtime's own staging, about 15 us behind the last kernel.)
-constexpr size_t HOST_RESULT_MAX = 1 << 20;
-class HostResult {
+// Pinned host memory that kernels on ctx().cur read small inputs from or write small results to
+// (read results after synchronising that stream).  A result in a device buffer copied to pageable
+// memory costs a copy kernel and the runtime's own staging, about 15 us behind the last kernel.
+constexpr size_t HOST_BLOCK_MAX = 1 << 20;  // callers use device buffers beyond this
+class HostBlock {
  public:
-  explicit HostResult(size_t bytes);
-  ~HostResult();
-  HostResult(const HostResult&) = delete;
-  HostResult& operator=(const HostResult&) = delete;
+  explicit HostBlock(size_t bytes);
+  ~HostBlock();
+  HostBlock(const HostBlock&) = delete;
+  HostBlock& operator=(const HostBlock&) = delete;
   template <class T>
   T* as() const {
     return static_cast<T*>(p_);

@@ -99,3 +99,28 @@ def test_oods_values(log_n, n_cols, n_points):
     for c in {0, n_cols // 2, n_cols - 1}:
         for k in range(n_points):
             assert got[k][c] == tuple(int(v) for v in O.eval_at_point(host[c], *pts[k])), (c, k)
+
+
+@pytest.mark.parametrize("log_n,n_cols,n_batches", [(1, 200, 1), (2, 17, 3), (5, 30, 2), (6, 13, 4), (7, 250, 1), (8, 16, 3),
+                                                    (9, 33, 4), (11, 70, 2), (12, 5, 3), (10, 700, 1),
+                                                    (9, 188, 1), (9, 190, 1), (4, 12400, 1)])
+def test_quotients_on_matrix_cores(log_n, n_cols, n_batches):
+    """Domains smaller than a wave's rows and larger than a block's, column counts that leave the
+    last step partly empty, one and two operand tiles, the sample counts at which the form
+    changes; extreme column values; a column sampled twice at one point."""
+    rng = np.random.default_rng(log_n * 1000 + n_cols)
+    host = [rng.integers(0, S.P, 1 << log_n, dtype=np.uint32) for _ in range(n_cols)]
+    host[0][:] = S.P - 1
+    cols = [S.BaseFieldVec.from_numpy(h) for h in host]
+    batches = []
+    for b in range(n_batches):
+        cs = [c for c in range(n_cols) if (c + b) % 3 != 1 or c == 0]
+        batches.append((S.random_circle_point_qm31(rng), [(c, S.random_qm31(rng)) for c in cs]))
+    batches[0][1].append((0, S.random_qm31(rng)))
+    rc = S.random_qm31(rng)
+    dom = S.canonic_half_coset(log_n)
+    out = S.SecureColumn.uninitialized(1 << log_n)
+    S.accumulate_quotients_async(dom, cols, rc, S.QuotientSamples(batches), out)
+    want = O.accumulate_quotients(dom.initial_index, dom.step_size, log_n, host, rc, batches)
+    assert (out.to_numpy() == want).all()
+    assert (S.accumulate_quotients(dom, cols, rc, batches).to_numpy() == want).all()
