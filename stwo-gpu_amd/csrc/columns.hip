@@ -9,6 +9,7 @@
 // brev(mid) exchange places as a bit-reversed transpose through LDS, with
 // 2^a-element contiguous runs on both the read and the write side.
 #include "field.hpp"
+#include "gmem.hpp"
 #include "runtime.hpp"
 
 namespace sh {
@@ -94,116 +95,118 @@ __global__ __launch_bounds__(BR_NT) void bitrev_tiled16_kernel(T* a, uint32_t lo
   }
 }
 
-// 4-byte elements in columns of at least 2^14: 128 x 128 tiles (512-byte runs; 2^28 values
-// 0.70 -> 0.61 ms against 64 x 64 tiles, 0.58 ms with two elements per 8-byte access), both
-// tiles of the pair in registers and one padded LDS tile for the two transposes
-template <class T, int TA, int NT>
-__global__ __launch_bounds__(NT) void bitrev_big_kernel(T* a, uint32_t log_n) {
-  constexpr uint32_t W = 1u << TA, RW = W + 1;
-  constexpr int PER = (int)(W * W / NT) / 2;  // element pairs per thread and tile
-  __shared__ T t[W * RW];
-  const uint32_t mid_bits = log_n - 2 * TA;
-  const uint32_t m = blockIdx.x;
-  const uint32_t mr = brev(m, mid_bits);
-  if (mr < m) return;
-  const bool pair = mr != m;
-  // pair e of a tile: row e >> (TA - 1), elements lo, lo + 1 with lo = 2 (e mod W / 2); one
-  // 8-byte access per pair, so a wave covers a whole 512-byte row
-  auto at2 = [&](uint32_t hi, uint32_t mid, uint32_t lo) -> size_t {
-    return (((size_t)hi << (log_n - TA)) | ((size_t)mid << TA) | lo) >> 1;
-  };
-  uint2* const a2 = reinterpret_cast<uint2*>(a);
-  uint2 va[PER], vb[PER];
-#pragma unroll
-  for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi = e >> (TA - 1), lo = 2 * (e & (W / 2 - 1));
-    va[k] = a2[at2(hi, m, lo)];
-    if (pair) vb[k] = a2[at2(hi, mr, lo)];
-  }
-#pragma unroll
-  for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi = e >> (TA - 1), lo = 2 * (e & (W / 2 - 1));
-    t[hi * RW + lo] = va[k].x;
-    t[hi * RW + lo + 1] = va[k].y;
-  }
-  __syncthreads();
-  // element (hi, m, lo) goes to (brev lo, mr, brev hi)
-#pragma unroll
-  for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi2 = e >> (TA - 1), lo2 = 2 * (e & (W / 2 - 1));
-    a2[at2(hi2, mr, lo2)] = make_uint2(t[brev(lo2, TA) * RW + brev(hi2, TA)], t[brev(lo2 + 1, TA) * RW + brev(hi2, TA)]);
-  }
-  if (!pair) return;
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi = e >> (TA - 1), lo = 2 * (e & (W / 2 - 1));
-    t[hi * RW + lo] = vb[k].x;
-    t[hi * RW + lo + 1] = vb[k].y;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi2 = e >> (TA - 1), lo2 = 2 * (e & (W / 2 - 1));
-    a2[at2(hi2, m, lo2)] = make_uint2(t[brev(lo2, TA) * RW + brev(hi2, TA)], t[brev(lo2 + 1, TA) * RW + brev(hi2, TA)]);
-  }
+// Tile of block b: neighbouring places of the XCD order alternate between steps of m's lowest and
+// of its highest bits, so the tiles that are under way together lie in runs both at m and at the
+// mirrored brev(m).
+__device__ __forceinline__ uint32_t mirrored_order(uint32_t mid_bits) {
+  const uint32_t b = xcd_order();
+  uint32_t m = 0;
+  for (uint32_t k = 0; k < mid_bits; k++) m |= ((b >> k) & 1u) << ((k & 1) ? mid_bits - 1 - k / 2 : k / 2);
+  return m;
 }
 
-// 16-byte elements in columns of at least 2^12: 64 x 64 tiles (1 KiB runs), both tiles of the
-// pair in registers; LDS row r starts at element 64 r + r / 8, so the transposed reads of 8
-// consecutive lanes (rows 8 apart) fall in distinct bank groups (with one element of padding
-// per row they all hit one group: 3.1 ms for 2^28, against 2.5 ms for 32 x 32 tiles and 2.17
-// ms here)
-__global__ __launch_bounds__(1024) void bitrev_big16_kernel(uint4* a, uint32_t log_n) {
-  constexpr uint32_t TA = 6, W = 1u << TA, NT = 1024;
-  constexpr int PER = (int)(W * W / NT);
-  __shared__ uint4 t[W * W + W / 8];
-  const uint32_t mid_bits = log_n - 2 * TA;
-  const uint32_t m = blockIdx.x;
-  const uint32_t mr = brev(m, mid_bits);
-  if (mr < m) return;
+// 4-byte elements in columns of at least 2^14: 128 x 128 tiles (512-byte runs), both tiles of the
+// pair in registers and one padded LDS tile for the two transposes.  A wave's 16-byte accesses
+// cover two rows.  Bound by the memory system: 2^28 values 591 -> 499 us (4.3 TB/s), where the
+// same exchange of tiles without the transposes takes 460 and a pass over the tiles in place 390.
+// 8 waves a block leave room for a second one beside it; 16 waves with 8-byte accesses, in the
+// order of m, took 585, 64 x 64 tiles 620 or more, 256 x 256 tiles do not leave room for two
+// blocks (780 for the exchange alone).
+template <bool NT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void bitrev_big_kernel(uint32_t* a,
+                                                                                                uint32_t log_n) {
+  constexpr uint32_t TA = 7, W = 1u << TA, RW = W + 1;
+  constexpr int PER = 8;  // 16-byte accesses per thread and tile
+  __shared__ uint32_t t[W * RW];
+  const uint32_t m = mirrored_order(log_n - 2 * TA), mr = brev(m, log_n - 2 * TA);
+  if (mr < m) return;  // the pair is handled by the block of mr
   const bool pair = mr != m;
-  auto at = [&](uint32_t hi, uint32_t mid, uint32_t lo) -> size_t {
-    return ((size_t)hi << (log_n - TA)) | ((size_t)mid << TA) | lo;
+  // a wave's access: rows hi, hi + 1 (a half wave each) of the tile, hi = 2 wave + 16 k
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), half = (threadIdx.x >> 5) & 1,
+                 l = threadIdx.x & 31;
+  const uint32_t off = (half << (log_n - TA)) + 4 * l;
+  typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(4)));
+  auto row = [&](uint32_t mm, int k) {
+    return (SH_GLOBAL u4*)((SH_GLOBAL char*)as_global(a + (((size_t)(2 * wave + 16 * k) << (log_n - TA)) | (mm << TA))) +
+                           off * 4u);
   };
-  auto row = [](uint32_t r) { return r * W + (r >> 3); };
-  // plain words in registers (arrays of the vector type would be kept in scratch memory)
-  uint32_t va[PER][4], vb[PER][4];
+  u4 va[PER], vb[PER];
 #pragma unroll
   for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi = e >> TA, lo = e & (W - 1);
-    const uint4 x = a[at(hi, m, lo)];
-    va[k][0] = x.x; va[k][1] = x.y; va[k][2] = x.z; va[k][3] = x.w;
-    if (pair) {
-      const uint4 y = a[at(hi, mr, lo)];
-      vb[k][0] = y.x; vb[k][1] = y.y; vb[k][2] = y.z; vb[k][3] = y.w;
+    va[k] = NT ? __builtin_nontemporal_load(row(m, k)) : *row(m, k);
+    if (pair) vb[k] = NT ? __builtin_nontemporal_load(row(mr, k)) : *row(mr, k);
+  }
+  uint32_t* const in = t + (2 * wave + half) * RW + 4 * l;
+  // element (hi, m, lo) goes to (brev lo, mr, brev hi): row hi = 16 k + 2 wave + half, column
+  // lo = 4 l + j of the result are column and row of the tile, reversed
+  const uint32_t* const out = t + brev(l, 5) * RW + (half << 6) + (brev(wave, 3) << 3);
+  auto turn = [&](const u4 (&v)[PER], uint32_t to) {
+#pragma unroll
+    for (int k = 0; k < PER; k++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) in[16 * RW * k + j] = v[k][j];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int c = (k & 1) << 2 | (k & 2) | k >> 2;
+      const u4 x = {out[c], out[64 * RW + c], out[32 * RW + c], out[96 * RW + c]};
+      if (NT)
+        __builtin_nontemporal_store(x, row(to, k));
+      else
+        *row(to, k) = x;
     }
-  }
-#pragma unroll
-  for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi = e >> TA, lo = e & (W - 1);
-    t[row(hi) + lo] = make_uint4(va[k][0], va[k][1], va[k][2], va[k][3]);
-  }
-  __syncthreads();
-  // element (hi, m, lo) goes to (brev lo, mr, brev hi)
-#pragma unroll
-  for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi2 = e >> TA, lo2 = e & (W - 1);
-    a[at(hi2, mr, lo2)] = t[row(brev(lo2, TA)) + brev(hi2, TA)];
-  }
+  };
+  turn(va, mr);
   if (!pair) return;
   __syncthreads();
+  turn(vb, m);
+}
+
+// 16-byte elements in columns of at least 2^12: 64 x 64 tiles (1 KiB runs), the same way; LDS row
+// r starts at element 64 r + r / 8, so the transposed reads of 8 consecutive lanes (rows 8 apart)
+// fall in distinct bank groups.  2^26 values 570 -> 469 us (4.6 TB/s).
+template <bool NT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) void bitrev_big16_kernel(uint4* a,
+                                                                                                  uint32_t log_n) {
+  constexpr uint32_t TA = 6, W = 1u << TA;
+  constexpr int PER = 8;  // elements per thread and tile
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  __shared__ u4 t[W * W + W / 8];
+  const uint32_t m = mirrored_order(log_n - 2 * TA), mr = brev(m, log_n - 2 * TA);
+  if (mr < m) return;  // the pair is handled by the block of mr
+  const bool pair = mr != m;
+  // a wave's access: row hi = wave + 8 k of the tile
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  auto row = [&](uint32_t mm, int k) {
+    return (SH_GLOBAL u4*)as_global(a + (((size_t)(wave + 8 * k) << (log_n - TA)) | (mm << TA))) + lane;
+  };
+  auto lds_row = [](uint32_t r) { return r * W + (r >> 3); };
+  u4 va[PER], vb[PER];
 #pragma unroll
   for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi = e >> TA, lo = e & (W - 1);
-    t[row(hi) + lo] = make_uint4(vb[k][0], vb[k][1], vb[k][2], vb[k][3]);
+    va[k] = NT ? __builtin_nontemporal_load(row(m, k)) : *row(m, k);
+    if (pair) vb[k] = NT ? __builtin_nontemporal_load(row(mr, k)) : *row(mr, k);
   }
+  u4* const in = t + wave * W + lane;
+  // element (hi, m, lo) goes to (brev lo, mr, brev hi)
+  const u4* const out = t + lds_row(brev(lane, TA)) + (brev(wave, 3) << 3);
+  auto turn = [&](const u4 (&v)[PER], uint32_t to) {
+#pragma unroll
+    for (int k = 0; k < PER; k++) in[8 * W * k + k] = v[k];  // (lds_row(wave + 8 k): wave is below 8)
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const u4 x = out[(k & 1) << 2 | (k & 2) | k >> 2];
+      if (NT)
+        __builtin_nontemporal_store(x, row(to, k));
+      else
+        *row(to, k) = x;
+    }
+  };
+  turn(va, mr);
+  if (!pair) return;
   __syncthreads();
-#pragma unroll
-  for (int k = 0; k < PER; k++) {
-    const uint32_t e = threadIdx.x + NT * k, hi2 = e >> TA, lo2 = e & (W - 1);
-    a[at(hi2, m, lo2)] = t[row(brev(lo2, TA)) + brev(hi2, TA)];
-  }
+  turn(vb, m);
 }
 
 template <class T>
@@ -218,6 +221,10 @@ __global__ void bitrev_simple_kernel(T* a, uint32_t n, uint32_t log_n) {
   }
 }
 
+// log of the 4-byte values from which the accesses are nontemporal (16-byte values: two less), the
+// column being larger than the caches.  Nontemporal / plain: 2^27 M31 253 / 280 us, 2^26 135 / 92;
+// 2^25 QM31 245 / 262, 2^24 138 / 95.
+constexpr uint32_t BR_STREAM = 27;
 template <class T>
 void bit_reverse(T* a, uint64_t n) {
   require(is_pow2(n) && n <= (1ull << 31), "bit_reverse: size must be a power of two <= 2^31");
@@ -226,12 +233,14 @@ void bit_reverse(T* a, uint64_t n) {
   if (log_n >= 2 * TA) {
     timed("bit_reverse", [&] {
       if constexpr (sizeof(T) == 4) {
-        if (log_n >= 14 && ((uintptr_t)a & 7) == 0)  // 8-byte accesses
-          bitrev_big_kernel<T, 7, 1024><<<1u << (log_n - 14), 1024, 0, ctx().cur>>>(a, log_n);
+        if (log_n >= 14)
+          (log_n >= BR_STREAM ? bitrev_big_kernel<true> : bitrev_big_kernel<false>)<<<1u << (log_n - 14), 512, 0,
+                                                                                       ctx().cur>>>(a, log_n);
         else
           bitrev_tiled_kernel<T><<<1u << (log_n - 2 * TA), cols::BR_NT, 0, ctx().cur>>>(a, log_n);
       } else if (log_n >= 12)
-        bitrev_big16_kernel<<<1u << (log_n - 12), 1024, 0, ctx().cur>>>(a, log_n);
+        (log_n >= BR_STREAM - 2 ? bitrev_big16_kernel<true> : bitrev_big16_kernel<false>)<<<1u << (log_n - 12), 512, 0,
+                                                                                         ctx().cur>>>(a, log_n);
       else
         bitrev_tiled16_kernel<T><<<1u << (log_n - 2 * TA), cols::BR_NT, 0, ctx().cur>>>(a, log_n);
     });

@@ -124,3 +124,17 @@ def test_quotients_on_matrix_cores(log_n, n_cols, n_batches):
     want = O.accumulate_quotients(dom.initial_index, dom.step_size, log_n, host, rc, batches)
     assert (out.to_numpy() == want).all()
     assert (S.accumulate_quotients(dom, cols, rc, batches).to_numpy() == want).all()
+
+
+@pytest.mark.parametrize("log_n", [13, 14, 15, 18])
+@pytest.mark.parametrize("offset", [1, 2, 3])
+def test_bit_reverse_at_word_aligned_columns(log_n, offset):
+    """Columns that start at any word: 16-byte accesses off their alignment, and nothing beyond the
+    column's ends touched."""
+    data = np.arange((1 << log_n) + 8, dtype=np.uint32)
+    col = S.BaseFieldVec.from_numpy(data)
+    S.lib().bit_reverse_base_field(col.ptr + 4 * offset, 1 << log_n)
+    S.check()
+    want = data.copy()
+    want[offset:offset + (1 << log_n)] = O.bit_reverse(data[offset:offset + (1 << log_n)].copy())
+    assert (col.to_numpy() == want).all()
