@@ -241,22 +241,23 @@ __device__ __forceinline__ qm31 leaf_fold_value(const LeafFold& lf, const uint32
 template <int NT>
 __device__ __forceinline__ void build_levels(const Hash* prev, uint32_t top, uint32_t depth, uint32_t nodes0,
                                              uint32_t base0, Hash* const* outs, const LayerCols* inj, Hash* s,
-                                             uint32_t (*qmsg)[16], uint64_t jo, const LeafFold& lf) {
+                                             bool staged, uint32_t (*qmsg)[16], uint64_t jo, const LeafFold& lf) {
   for (uint32_t d = 0; d < depth; d++) {
     const uint32_t layer = top - d;
     const uint32_t cnt = nodes0 >> d;
     const uint32_t base = base0 >> d;
     const LayerCols lc = ld_uniform(inj, layer);
-    SH_GLOBAL Hash* const out = as_global(jptr(outs[layer], jo));
+    SH_GLOBAL Hash* const out = as_global(jptr(ld_uniform(outs, layer), jo));
     // the leaf level of a LeafFold launch: four columns, computed here (prev is null)
     const bool fold = d == 0 && lf.src[0] != nullptr;
-    if ((d > 0 || !prev) && cnt <= NT / 4) {
+    const bool in_s = d > 0 || staged;  // the children are in s
+    if ((in_s || !prev) && cnt <= NT / 4) {
       // narrow level: one quad per node, children read from s in place (a leaf level of at
       // most NT / 4 nodes too: it has no children, only its columns)
       const uint32_t i = threadIdx.x >> 2, q = threadIdx.x & 3;
       uint32_t h_lo = 0, h_hi = 0;
       if (i < cnt) {
-        if (d > 0) quad_compress(h_lo, h_hi, s[2 * i].s, q);
+        if (in_s) quad_compress(h_lo, h_hi, s[2 * i].s, q);
         uint32_t* mb = qmsg[i];
         if (fold) {
           // each lane of the quad folds the leaf, stores its own coordinate and stages it
@@ -295,9 +296,9 @@ __device__ __forceinline__ void build_levels(const Hash* prev, uint32_t top, uin
       const uint32_t i = r0 + threadIdx.x;
       uint32_t h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
       if (i < cnt) {
-        if (d > 0 || prev) {  // leaves (no prev) have no children to compress
+        if (in_s || prev) {  // leaves (no prev) have no children to compress
           uint32_t m[16];
-          if (d == 0) {
+          if (!in_s) {
             load_children(as_global(prev), base + i, m);
           } else {
 #pragma unroll
@@ -335,6 +336,12 @@ __device__ __forceinline__ void build_levels(const Hash* prev, uint32_t top, uin
 // chip.  No block waits for another: each block publishes its nodes (device-scope fence)
 // and counts itself in; the block that counts last continues, the others exit.  The last
 // block resets the counter for the next launch.
+// What such a launch costs beside its levels (a compression of a quad is 0.7 us) is the hand-over:
+// the counting side only releases and the last block only acquires (a full fence on both sides
+// writes the XCD's L2 back twice), the block roots go to LDS so that quads hash them (a lane's
+// compression takes 1.6 us), and both passes run one copy of the code, which the last block then
+// has in its instruction cache.  2^12 leaves of one QM31 column: 25.5 -> 21 us (28 -> 24 with the
+// fold and the channel step).
 constexpr uint32_t SUB_BLOCK_LOG = 7;  // nodes per block at the top layer (one lane quad each below)
 // Runs topped by at most 2^12 nodes (at most 32 blocks) finish in their last block.  The
 // device-scope fence of every block writes its XCD's L2 back, which costs more than a
@@ -350,7 +357,7 @@ template <int NT>
 __global__ __launch_bounds__(NT) void subtree_kernel(const Hash* prev, uint32_t top, uint32_t depth, uint32_t w_log,
                                                      Hash* const* outs, const LayerCols* inj, RootDraw rd,
                                                      uint32_t* arrive, uint64_t js, LeafFold lf) {
-  extern __shared__ Hash s[];  // max(2^w_log, block count / 2) hashes
+  extern __shared__ __align__(16) Hash s[];  // max(2^(w_log + 1), block count) hashes
   __shared__ uint32_t qmsg[NT / 4][16];  // quad mode: staging of injected column chunks
   __shared__ uint32_t is_last;
   // batched jobs (blockIdx.z): every arena pointer moves by the job's offset; one arrival
@@ -362,19 +369,35 @@ __global__ __launch_bounds__(NT) void subtree_kernel(const Hash* prev, uint32_t 
     rd.ch = jptr(rd.ch, jo);
     rd.dst = jptr(rd.dst, jo);
   }
-  const uint32_t bd = arrive ? w_log + 1 : depth;  // levels built by every block
-  build_levels<NT>(prev, top, bd, 1u << w_log, blockIdx.x << w_log, outs, inj, s, qmsg, jo, lf);
-  if (arrive) {
-    __threadfence();  // this block's nodes are visible device-wide before it counts in
+  // first the levels of this block; then, in the last block, those above every block's root (a loop,
+  // so that the second pass finds its code in the instruction cache)
+  uint32_t n_levels = arrive ? w_log + 1 : depth, nodes = 1u << w_log, base = blockIdx.x << w_log, layer = top;
+  LeafFold fold = lf;
+  // children of a first level that quads hash: copied to s
+  bool staged = false;
+  auto stage = [&](const Hash* from, uint32_t n) {
+    const SH_GLOBAL uint4* const w = (const SH_GLOBAL uint4*)as_global(from);
+    for (uint32_t t = threadIdx.x; t < 2 * n; t += NT) reinterpret_cast<uint4*>(s)[t] = w[t];
+    __syncthreads();
+    staged = true;
+  };
+  if (prev && nodes <= NT / 4) stage(prev + 2 * (size_t)base, 2 * nodes);
+  for (bool last = false;; last = true) {
+    build_levels<NT>(prev, layer, n_levels, nodes, base, outs, inj, s, staged, qmsg, jo, fold);
+    if (!arrive || last) break;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // this block's nodes are visible before it counts in
     __syncthreads();
     if (threadIdx.x == 0) is_last = atomicAdd(arrive, 1u) == gridDim.x - 1 ? 1u : 0u;
     __syncthreads();
     if (!is_last) return;  // uniform over the block
-    __threadfence();       // every other block's nodes are visible to the loads below
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // every block's nodes are visible to the loads below
     if (threadIdx.x == 0) *arrive = 0u;
-    const uint32_t t_top = top - bd;  // the block roots are layer t_top + 1
-    build_levels<NT>(jptr(outs[t_top + 1], jo), t_top, depth - bd, gridDim.x >> 1, 0, outs, inj, s, qmsg, jo,
-                     LeafFold{});
+    layer = top - n_levels;  // the block roots are layer + 1
+    stage(jptr(ld_uniform(outs, layer + 1), jo), gridDim.x);
+    n_levels = depth - n_levels;
+    nodes = gridDim.x >> 1;
+    base = 0;
+    fold.src[0] = nullptr;
   }
   // the launch that wrote the root (layer 0, held in s[0] after the last barrier) runs
   // the channel step on one lane quad: Channel::mix8 and Channel::draw_qm31 / draw_point
@@ -521,7 +544,7 @@ bool MerklePlan::enqueue_from(size_t* next, uint32_t min_layer, const std::vecto
       const uint32_t blocks = 1u << (s.top - w_log);
       const bool tail = s.depth > w_log + 1;
       require(!tail || (narrow && blocks >= 2), "merkle: bad subtree step");
-      const size_t lds = sizeof(Hash) * std::max<size_t>(1u << w_log, tail ? blocks / 2 : 0);
+      const size_t lds = sizeof(Hash) * std::max<size_t>(2u << w_log, tail ? blocks : 0);
       // the launch that writes the root also runs the channel step
       RootDraw rd{nullptr, nullptr, 0};
       if (root_draw && s.top + 1 == s.depth) {

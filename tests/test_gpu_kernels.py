@@ -138,3 +138,19 @@ def test_bit_reverse_at_word_aligned_columns(log_n, offset):
     want = data.copy()
     want[offset:offset + (1 << log_n)] = O.bit_reverse(data[offset:offset + (1 << log_n)].copy())
     assert (col.to_numpy() == want).all()
+
+
+@pytest.mark.parametrize("sizes", [[k] * 4 for k in range(15)] + [[16] * 20 + [15, 7], [17] * 4 + [16, 8, 7, 7, 6],
+                                                                  [12] * 4 + [7] * 3 + [5] + [4] * 2, [9] * 17 + [8, 0]])
+def test_merkle_subtree_launches(sizes):
+    """Trees of every height that one or two subtree launches build: launches whose last block goes on
+    above the other blocks' roots, and launches that start from another launch's nodes, with columns
+    injected at their first level and above.  Twice: the arrival counters are left as they were."""
+    rng = np.random.default_rng(sum(sizes) + len(sizes))
+    host = [rng.integers(0, S.P, 1 << k, dtype=np.uint32) for k in sizes]
+    cols = [S.BaseFieldVec.from_numpy(h) for h in host]
+    want = O.merkle_commit(host)
+    for _ in range(2):
+        tree = S.MerkleTree(cols).commit_async()
+        for k, layer in enumerate(tree.layers):
+            assert (layer.to_numpy().reshape(-1) == want[k].reshape(-1)).all(), k
