@@ -154,3 +154,30 @@ def test_merkle_subtree_launches(sizes):
         tree = S.MerkleTree(cols).commit_async()
         for k, layer in enumerate(tree.layers):
             assert (layer.to_numpy().reshape(-1) == want[k].reshape(-1)).all(), k
+
+
+@pytest.mark.parametrize("n", [1, 255, 2049, 1 << 20, (1 << 24) - 3, (1 << 24) + 1])
+def test_batch_inverse_secure_field_sizes(n):
+    """Sizes at which the kernel changes and blocks end; extreme values and zeros among the inputs."""
+    rng = np.random.default_rng(n)
+    data = rng.integers(0, S.P, (n, 4), dtype=np.uint32)
+    for k, row in enumerate([(0, 0, 0, 0), (S.P - 1,) * 4, (0, 0, S.P - 1, 1), (0, S.P - 1, 0, 0), (1, 0, 0, 0)]):
+        data[(k * 37) % n] = row
+    dst = S.SecureFieldVec.uninitialized(n)
+    S.batch_inverse(S.SecureFieldVec.from_numpy(data), dst)
+    got = dst.to_numpy().reshape(-1, 4)
+    # x * (1 / x) = 1, in 64 bits: (a + b u)(c + d u) with u^2 = R = 2 + i over CM31
+    P = np.uint64(S.P)
+
+    def cm(x, y):
+        return ((x[0] * y[0] % P + (P - x[1] * y[1] % P)) % P, (x[0] * y[1] % P + x[1] * y[0] % P) % P)
+
+    x, y = data.astype(np.uint64).T, got.astype(np.uint64).T
+    xx, yy = cm(x[:2], y[:2]), cm(x[2:], y[2:])
+    xy, yx = cm(x[:2], y[2:]), cm(x[2:], y[:2])
+    r = ((P + P + yy[0] + yy[0] - yy[1]) % P, (yy[0] + yy[1] + yy[1]) % P)
+    prod = [(xx[0] + r[0]) % P, (xx[1] + r[1]) % P, (xy[0] + yx[0]) % P, (xy[1] + yx[1]) % P]
+    zero = (data == 0).all(axis=1)
+    assert (prod[0] == np.where(zero, 0, 1)).all()
+    assert all((p == 0).all() for p in prod[1:])
+    assert (got[zero] == 0).all()
