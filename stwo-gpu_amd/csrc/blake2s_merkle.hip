@@ -611,7 +611,6 @@ extern "C" int stwo_hip_merkle_commit_async(uint32_t n_cols, const uint32_t* con
 
 extern "C" int stwo_hip_merkle_root(const StwoBlake2sHash* root_layer, StwoBlake2sHash* root_out) {
   return guarded([&] {
-    hip_check(hipMemcpyAsync(root_out, root_layer, 32, hipMemcpyDefault, ctx().cur), "hipMemcpy");
-    sync();
+    download(root_out, root_layer, 32);
   });
 }

@@ -248,6 +248,43 @@ HostBlock::~HostBlock() {
   st.held = false;
 }
 
+// Small results to host memory, waiting for them: a kernel behind the one that wrote them copies
+// to pinned memory (bytes a multiple of 4).  The runtime's copy to pageable memory starts its own
+// kernel late and stages the result again: a root of 32 bytes FIGURE.
+__global__ void download_kernel(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, uint32_t n4) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n4) dst[i] = src[i];
+}
+constexpr size_t DOWNLOAD_KERNEL_MAX = 1 << 16;
+// whether the bytes at src lie in one allocation of this device and dst is ordinary host memory
+// (any other pair of pointers goes to the runtime, to be copied or refused)
+static bool device_to_host(const void* dst, const void* src, size_t bytes) {
+  hipPointerAttribute_t s{}, d{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  const bool ok = hipPointerGetAttributes(&s, src) == hipSuccess && s.type == hipMemoryTypeDevice &&
+                  s.device == g_ctx.device && hipMemGetAddressRange(&base, &size, const_cast<void*>(src)) == hipSuccess &&
+                  (const char*)src + bytes <= (const char*)base + size &&
+                  hipPointerGetAttributes(&d, dst) == hipSuccess && d.type == hipMemoryTypeUnregistered;
+  if (!ok) (void)hipGetLastError();  // (a pointer that the runtime does not know is no error here)
+  return ok;
+}
+void download(void* host, const void* dev, size_t bytes) {
+  if (!bytes) return;
+  if (bytes > DOWNLOAD_KERNEL_MAX || bytes % 4 || (uintptr_t)dev % 4 || g_ctx.cur != g_ctx.stream ||
+      !device_to_host(host, dev, bytes)) {
+    hip_check(hipMemcpyAsync(host, dev, bytes, hipMemcpyDefault, g_ctx.cur), "hipMemcpy");
+    sync();
+    return;
+  }
+  Staging& st = take_staging(bytes);
+  const uint32_t n4 = (uint32_t)(bytes / 4);
+  download_kernel<<<(n4 + 255) / 256, 256, 0, g_ctx.cur>>>((uint32_t*)st.host, (const uint32_t*)dev, n4);
+  hip_check(hipGetLastError(), "download_kernel");
+  sync();
+  memcpy(host, st.host, bytes);  // (the buffer is free again: nothing else was taken meanwhile)
+}
+
 DevBuf upload(const void* host, size_t bytes) {
   DevBuf b(bytes);
   upload_to(b.p, host, bytes);
@@ -306,8 +343,7 @@ extern "C" int stwo_hip_free(void* ptr) {
 }
 extern "C" int stwo_hip_memcpy(void* dst, const void* src, size_t bytes) {
   return guarded([&] {
-    hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, ctx().stream), "hipMemcpy");
-    sync();
+    download(dst, src, bytes);
   });
 }
 extern "C" int stwo_hip_release_cached_memory(void) {
@@ -368,9 +404,7 @@ extern "C" int stwo_hip_kernel_stats_reset(void) {
 // C ABI: reference memory functions (bindings.rs:77-99, 196-216)
 // =========================================================================
 static void copy_sync(void* dst, const void* src, size_t bytes) {
-  if (!bytes) return;
-  hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, ctx().stream), "hipMemcpy");
-  sync();
+  download(dst, src, bytes);
 }
 
 extern "C" void copy_uint32_t_vec_from_device_to_host(const uint32_t* device_ptr, uint32_t* host_ptr,

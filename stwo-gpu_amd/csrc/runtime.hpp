@@ -141,6 +141,9 @@ struct DevBuf {
 DevBuf upload(const void* host, size_t bytes);
 // Same into existing device memory.
 void upload_to(void* dev, const void* host, size_t bytes);
+// A copy between any two pointers on the current stream that is complete on return; made for small
+// results in host memory.
+void download(void* dst, const void* src, size_t bytes);
 
 // Pinned host memory that kernels on ctx().cur read small inputs from or write small results to
 // (read results after synchronising that stream).  A result in a device buffer copied to pageable
