@@ -24,7 +24,12 @@ namespace tw {
 // 2^z, one of levels 12 + 1 .. 12 + z.  Bound by the latency of the products and of the
 // doublings (2^22: 103 -> 13.8 us against a full power of the step per entry, which took 2 x 31
 // products each; the stores alone take 3 us).
-constexpr uint32_t TREE_BLOCK_LOG = 12, TREE_NT = 256;
+constexpr uint32_t TREE_NT = 256;
+// Blocks of 2^12 values, or of 2^10: a quarter of the chain of products and doublings and four times
+// the blocks, for trees up to 2^20 (a call with the inverses: 2^14 25.2 us with the small blocks, 28.3
+// with the large; 2^20 28.5 / 31.2; 2^21 33.6 / 33.4; 2^22 43.6 / 39.5; a power per entry took 25.4,
+// 46, 70 and 120).
+constexpr uint32_t TREE_SMALL_MAX = 20;
 
 struct TreeArgs {
   pt initial;
@@ -32,29 +37,36 @@ struct TreeArgs {
   pt lane16[16];  // sum of the weights of bits 0, 1, 10, 11 selected by the index's bits
 };
 
+template <uint32_t BLOCK_LOG>
 __global__ __launch_bounds__(TREE_NT) void tree_kernel(uint32_t* __restrict__ out, TreeArgs A, uint32_t log_size) {
   const uint32_t size = 1u << log_size, half_log = log_size - 1, half = size >> 1;  // log_size >= 1
   const uint32_t t = threadIdx.x, blk = blockIdx.x;
   if (blk == 0 && t == 0) out[size - 1] = 1;
   pt q = A.initial;
-  for (uint32_t b = TREE_BLOCK_LOG; b < half_log; b++)  // uniform
-    if ((blk >> (b - TREE_BLOCK_LOG)) & 1) q = pmul(q, A.weight[b]);
+  for (uint32_t b = BLOCK_LOG; b < half_log; b++)  // uniform
+    if ((blk >> (b - BLOCK_LOG)) & 1) q = pmul(q, A.weight[b]);
 #pragma unroll
   for (int b = 0; b < 8; b++) {
+    if (b + 2 >= (int)half_log) break;  // uniform: a small tree has fewer index bits
     const pt r = pmul(q, A.weight[b + 2]);
     if ((t >> b) & 1) q = r;
   }
-  // value c of group k: index i = blk 2^12 + 2^10 k + 4 t + c
-  uint32_t x[4][4];
+  // value c of group k: index i = blk 2^12 + 2^10 k + 4 t + c (a small tree has fewer groups)
+  constexpr int GROUPS = 1 << (BLOCK_LOG - 10);
+  const uint32_t groups = min((uint32_t)GROUPS, (half + 1023) >> 10);
+  uint32_t x[GROUPS][4];
 #pragma unroll
-  for (int k = 0; k < 4; k++)
+  for (int k = 0; k < GROUPS; k++) {
+    if (k >= (int)groups) break;  // uniform, here and below
 #pragma unroll
     for (int c = 0; c < 4; c++) x[k][c] = pmul(q, A.lane16[4 * k + c]).x;
+  }
   auto twice = [](uint32_t v) { return sub(canon(2 * sqr(v)), 1); };
   // level j starts at size - (size >> j); j <= 2: 4, 2, 1 values per thread and group
 #pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const uint32_t i = (blk << TREE_BLOCK_LOG) + (k << 10) + 4 * t;
+  for (int k = 0; k < GROUPS; k++) {
+    if (k >= (int)groups) break;
+    const uint32_t i = (blk << BLOCK_LOG) + (k << 10) + 4 * t;
 #pragma unroll
     for (int j = 0; j < 3; j++) {
       uint32_t* lvl = out + (size - (size >> j));
@@ -71,8 +83,9 @@ __global__ __launch_bounds__(TREE_NT) void tree_kernel(uint32_t* __restrict__ ou
     if (j >= log_size) return;  // uniform
     uint32_t* lvl = out + (size - (size >> j));
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const uint32_t i = (blk << TREE_BLOCK_LOG) + (k << 10) + 4 * t;
+    for (int k = 0; k < GROUPS; k++) {
+      if (k >= (int)groups) break;
+      const uint32_t i = (blk << BLOCK_LOG) + (k << 10) + 4 * t;
       if ((t & ((1u << (j - 2)) - 1)) == 0 && i < half) lvl[i >> j] = x[k][0];
       x[k][0] = twice(x[k][0]);
     }
@@ -83,12 +96,13 @@ __global__ __launch_bounds__(TREE_NT) void tree_kernel(uint32_t* __restrict__ ou
   for (uint32_t j = 10; j < log_size; j++) {
     uint32_t* lvl = out + (size - (size >> j));
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      const uint32_t i = (blk << TREE_BLOCK_LOG) + (k << 10);
+    for (int k = 0; k < GROUPS; k++) {
+      if (k >= (int)groups) break;
+      const uint32_t i = (blk << BLOCK_LOG) + (k << 10);
       if ((i & ((1u << j) - 1)) == 0 && i < half) lvl[i >> j] = x[k][0];
       x[k][0] = twice(x[k][0]);
     }
-    if (j >= TREE_BLOCK_LOG && (blk & ((2u << (j - TREE_BLOCK_LOG)) - 1))) return;
+    if (j >= BLOCK_LOG && (blk & ((2u << (j - BLOCK_LOG)) - 1))) return;
   }
 }
 
@@ -105,15 +119,16 @@ void compute_tree(uint32_t* out, pt initial, pt step, uint32_t log_size) {
   pt w = step;
   for (uint32_t b = 0; b < 30; b++) A.weight[b] = pt{1, 0};
   for (uint32_t b = half_log; b-- > 0; w = pmul(w, w)) A.weight[b] = w;  // weight[half_log - 1] = step
-  for (uint32_t s = 0; s < 16; s++) {
-    const uint32_t bit[4] = {0, 1, 10, 11};
-    pt r = {1, 0};
-    for (int b = 0; b < 4; b++)
-      if ((s >> b) & 1) r = pmul(r, A.weight[bit[b]]);
-    A.lane16[s] = r;
-  }
-  const uint32_t blocks = half_log > TREE_BLOCK_LOG ? 1u << (half_log - TREE_BLOCK_LOG) : 1u;
-  timed("twiddle_tree", [&] { tree_kernel<<<blocks, TREE_NT, 0, ctx().cur>>>(out, A, log_size); });
+  A.lane16[0] = pt{1, 0};
+  const uint32_t bit[4] = {0, 1, 10, 11};
+  for (uint32_t b = 0; b < 4; b++)
+    for (uint32_t s = 0; s < (1u << b); s++)
+      A.lane16[s + (1u << b)] = bit[b] < half_log ? pmul(A.lane16[s], A.weight[bit[b]]) : A.lane16[s];
+  const uint32_t block_log = log_size <= TREE_SMALL_MAX ? 10 : 12;
+  const uint32_t blocks = half_log > block_log ? 1u << (half_log - block_log) : 1u;
+  timed("twiddle_tree", [&] {
+    (block_log == 10 ? tree_kernel<10> : tree_kernel<12>)<<<blocks, TREE_NT, 0, ctx().cur>>>(out, A, log_size);
+  });
 }
 
 }  // namespace tw

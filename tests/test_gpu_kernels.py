@@ -8,7 +8,7 @@ import oracle as O  # noqa: E402
 import stwo_hip as S  # noqa: E402
 
 
-@pytest.mark.parametrize("log_n", [0, 1, 2, 3, 4, 9, 10, 11, 12, 13, 14, 17])
+@pytest.mark.parametrize("log_n", [0, 1, 2, 3, 4, 9, 10, 11, 12, 13, 14, 17, 20, 21, 22])
 @pytest.mark.parametrize("start", [1, 3, 0x155])
 def test_twiddle_tree_levels(log_n, start):
     """One block writes 2^12 values of level 0 and every level above them: sizes below, at and past
