@@ -181,3 +181,24 @@ def test_batch_inverse_secure_field_sizes(n):
     assert (prod[0] == np.where(zero, 0, 1)).all()
     assert all((p == 0).all() for p in prod[1:])
     assert (got[zero] == 0).all()
+
+
+@pytest.mark.parametrize("words,offset", [(1, 0), (1, 3), (255, 1), (257, 0), (1 << 14, 0), ((1 << 14) + 1, 2), (1 << 16, 1)])
+def test_copies_to_host_memory(words, offset):
+    """Either side of the size up to which a kernel copies, at any word of a buffer, right behind the
+    work that wrote it; and copies whose ends are other kinds of memory."""
+    data = np.arange(words + offset, dtype=np.uint32) * np.uint32(2654435761)
+    col = S.BaseFieldVec.from_numpy(data)
+    out = np.zeros(words + 1, np.uint32)
+    S.lib().copy_uint32_t_vec_from_device_to_host(col.ptr + 4 * offset, out.ctypes.data, words)
+    S.check()
+    assert (out[:words] == data[offset:]).all() and out[words] == 0
+    other = S.BaseFieldVec.uninitialized(words)
+    S.check(S.lib().stwo_hip_memcpy(other.ptr, col.ptr + 4 * offset, 4 * words))
+    back = np.zeros(words, np.uint32)
+    S.check(S.lib().stwo_hip_memcpy(back.ctypes.data, other.ptr, 4 * words))
+    assert (back == data[offset:]).all()
+    S.check(S.lib().stwo_hip_memcpy(other.ptr, data.ctypes.data, 4 * words))
+    assert (other.to_numpy() == data[:words]).all()
+    S.check(S.lib().stwo_hip_memcpy(back.ctypes.data, data.ctypes.data, 4 * words))
+    assert (back == data[:words]).all()
