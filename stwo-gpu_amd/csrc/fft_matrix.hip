@@ -493,14 +493,6 @@ __global__ __launch_bounds__(LT) void lde_matrix_kernel(StridedArgs A) {
 }
 
 // ---- host ------------------------------------------------------------------------
-// Column groups per block: a block's first group waits for its matrices and values with nothing
-// to compute, so blocks are as few as fill the chip a few times (256 columns of log 21, `fill`
-// 512 blocks at a time: 4 / 8 / 16 / 32 groups per block 1.09 / 1.04 / 0.99 / 0.99 ms).
-static uint32_t groups_per_block(uint64_t n_groups, uint64_t tiles, uint32_t fill) {
-  const uint64_t n = n_groups * tiles / (4ull * fill);
-  return (uint32_t)std::min<uint64_t>(32, std::max<uint64_t>(1, n));
-}
-
 // matrices of one direction over a domain of log_n: layers 4..7, 8..(contig - 1), then (strided
 // layers k > 0) 12..15 and 16..(11 + k)
 struct Tables {
