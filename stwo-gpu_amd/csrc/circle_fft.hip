@@ -721,16 +721,9 @@ static void launch_pass(const PassPlan& p, const PassArgs& base) {
   });
 }
 
-// the matrix-core kernels for small columns take blowups 1 .. 8
-static bool use_matrices_evaluate(uint32_t src_log, uint32_t log_n, uint64_t n_cols) {
-  return src_log + 3 >= log_n && use_matrices_tile(log_n, n_cols);
-}
-// Device memory for the matrices of a transform of whole small columns (0: none are used).
-static size_t tile_workspace_bytes(uint32_t log_n, uint64_t n_cols) {
-  return use_matrices_tile(log_n, n_cols) ? tile_matrix_bytes(log_n) : 0;
-}
-// The matrices of a transform of n_cols whole columns over the domain of log_n, when it uses
-// them: enqueued before the pointer tables are uploaded, so they are made while the host copies.
+// The matrices of a transform of whole small columns over the domain of log_n, when it uses them
+// (use_matrices_tile): enqueued before the pointer tables are uploaded, so they are made while the
+// host copies.
 static DevBuf tile_workspace(bool inverse, bool used, uint32_t log_n, const uint32_t* tw, uint64_t tree_len) {
   if (!used || tree_len < (1ull << (log_n - 1))) return DevBuf();  // (a short tree is refused later)
   DevBuf ws(tile_matrix_bytes(log_n));
@@ -740,8 +733,8 @@ static DevBuf tile_workspace(bool inverse, bool used, uint32_t log_n, const uint
 
 // Inverse FFT of n_cols columns of one log size (device pointer tables): the first pass
 // reads d_src, every pass writes d_cols (d_src == d_cols: in place).
-// ws: tile_workspace_bytes of device memory (may be null where that is 0), where the matrices
-// are already when ws_filled.
+// ws: tile_matrix_bytes of device memory for the matrix cores to take whole small columns (log 10 ..
+// 12; the matrices are there already when ws_filled), null for butterflies.
 void interpolate_same_size(uint32_t* const* d_cols, uint32_t n_cols, uint32_t log_n, const uint32_t* itw,
                            uint64_t tree_len, const uint32_t* const* d_src, uint32_t kc, void* ws, bool ws_filled = false) {
   require(log_n >= 1 && log_n <= 30, "interpolate: log size out of range");
@@ -752,7 +745,7 @@ void interpolate_same_size(uint32_t* const* d_cols, uint32_t n_cols, uint32_t lo
     });
     return;
   }
-  if (use_matrices_tile(log_n, n_cols)) {
+  if (ws) {
     const uint32_t* t = itw + (tree_len - (1ull << (log_n - 1)));
     if (!ws_filled) tile_matrices(true, log_n, t, (unsigned char*)ws);
     interpolate_tiles(d_src, d_cols, n_cols, log_n, t, (unsigned char*)ws);
@@ -775,7 +768,7 @@ void interpolate_same_size(uint32_t* const* d_cols, uint32_t n_cols, uint32_t lo
 }
 
 // Forward FFT: src columns (2^src_log coefficients) evaluated on the canonic domain
-// of log_n >= src_log, written to dst (device pointer tables).
+// of log_n >= src_log, written to dst (device pointer tables); ws as above, for log_n - src_log <= 3.
 void evaluate_same_size(uint32_t* const* d_dst, const uint32_t* const* d_src, uint32_t n_cols, uint32_t src_log,
                         uint32_t log_n, const uint32_t* tw, uint64_t tree_len, uint32_t kc, void* ws,
                         bool ws_filled = false) {
@@ -787,7 +780,7 @@ void evaluate_same_size(uint32_t* const* d_dst, const uint32_t* const* d_src, ui
     });
     return;
   }
-  if (use_matrices_evaluate(src_log, log_n, n_cols)) {
+  if (ws) {
     const uint32_t* t = tw + (tree_len - (1ull << (log_n - 1)));
     if (!ws_filled) tile_matrices(false, log_n, t, (unsigned char*)ws);
     evaluate_tiles(d_src, d_dst, n_cols, src_log, log_n, t, (unsigned char*)ws);
@@ -822,7 +815,9 @@ static void launch_lde_strided(uint32_t blocks, const PassArgs& Ai, const PassAr
 
 size_t lde_workspace_bytes(uint32_t n, uint32_t log_blowup, uint64_t n_cols, LdeVariant var) {
   if (var.mat && n >= 17 && n <= 20) return lde_matrix_bytes(n, log_blowup);
-  return std::max(tile_workspace_bytes(n, n_cols), tile_workspace_bytes(n + log_blowup, n_cols));
+  const size_t inv = use_matrices_tile(n, n_cols, true, 0, false) ? tile_matrix_bytes(n) : 0;
+  const size_t fwd = use_matrices_tile(n + log_blowup, n_cols, false, log_blowup, false) ? tile_matrix_bytes(n + log_blowup) : 0;
+  return std::max(inv, fwd);
 }
 
 // Interpolate d_src (2^n evaluations) into d_coeffs and evaluate on the canonic domain of
@@ -841,8 +836,10 @@ void lde_same_size(const uint32_t* const* d_src, uint32_t* const* d_coeffs, uint
   if (!var.fused || n < 14 || n > 12 + KS_MAX) {
     const uint32_t kci = (var.kc == 13 && n >= 14 && n - 13 <= KS_MAX) ? 13 : 0;
     const uint32_t kcf = (var.kc == 13 && m >= 14 && m - 13 <= KS_MAX) ? 13 : 0;
-    interpolate_same_size(d_coeffs, n_cols, n, itw, tree_len, d_src, kci, ws);
-    evaluate_same_size(d_lde, (const uint32_t* const*)d_coeffs, n_cols, n, m, tw, tree_len, kcf, ws);
+    interpolate_same_size(d_coeffs, n_cols, n, itw, tree_len, d_src, kci,
+                          use_matrices_tile(n, n_cols, true, 0, false) ? ws : nullptr);
+    evaluate_same_size(d_lde, (const uint32_t* const*)d_coeffs, n_cols, n, m, tw, tree_len, kcf,
+                       use_matrices_tile(m, n_cols, false, log_blowup, false) ? ws : nullptr);
     return;
   }
   const uint32_t k = n - 12, t = (k <= 8 ? 13 : BS_LDE) - k;
@@ -919,7 +916,8 @@ void lde_mixed(const uint32_t* const* src, uint32_t* const* coeffs, uint32_t* co
 // table is uploaded as it is, once when the columns are transformed in place.
 static void interpolate_one_size(uint32_t* const* cols, uint32_t n_cols, uint32_t log_n, const uint32_t* itw,
                                  uint64_t tree_len, const uint32_t* const* src) {
-  DevBuf ws = tile_workspace(true, use_matrices_tile(log_n, n_cols), log_n, itw, tree_len);
+  const bool in_place = !src || std::equal(src, src + n_cols, (const uint32_t* const*)cols);
+  DevBuf ws = tile_workspace(true, use_matrices_tile(log_n, n_cols, true, 0, in_place), log_n, itw, tree_len);
   DevBuf table = upload(cols, (size_t)n_cols * sizeof(void*));
   DevBuf stable = src ? upload(src, (size_t)n_cols * sizeof(void*)) : DevBuf();
   interpolate_same_size(table.as<uint32_t*>(), n_cols, log_n, itw, tree_len,
@@ -941,7 +939,7 @@ void interpolate_mixed(uint32_t* const* cols, const uint32_t* logs, uint32_t n_c
     size_t n = kv.second.first.size();
     DevBuf table = upload(kv.second.first.data(), n * sizeof(void*));
     DevBuf stable = upload(kv.second.second.data(), n * sizeof(void*));
-    DevBuf ws = tile_workspace(true, use_matrices_tile(kv.first, n), kv.first, itw, tree_len);
+    DevBuf ws = tile_workspace(true, use_matrices_tile(kv.first, n, true, 0, !src), kv.first, itw, tree_len);
     interpolate_same_size(table.as<uint32_t*>(), (uint32_t)n, kv.first, itw, tree_len,
                           stable.as<const uint32_t*>(), 0, ws.p, true);
   }
@@ -953,7 +951,8 @@ void evaluate_mixed(const uint32_t* const* src, const uint32_t* src_logs, uint32
   if (n_cols && std::all_of(src_logs, src_logs + n_cols, [&](uint32_t l) { return l == src_logs[0]; }) &&
       std::all_of(dst_logs, dst_logs + n_cols, [&](uint32_t l) { return l == dst_logs[0]; })) {
     const bool in_place = std::equal(src, src + n_cols, (const uint32_t* const*)dst);
-    DevBuf ws = tile_workspace(false, use_matrices_evaluate(src_logs[0], dst_logs[0], n_cols), dst_logs[0], tw, tree_len);
+    const uint32_t m = dst_logs[0], blowup = m - src_logs[0];
+    DevBuf ws = tile_workspace(false, use_matrices_tile(m, n_cols, false, blowup, in_place), m, tw, tree_len);
     DevBuf td = upload(dst, (size_t)n_cols * sizeof(void*));
     DevBuf ts = in_place ? DevBuf() : upload(src, (size_t)n_cols * sizeof(void*));
     evaluate_same_size(td.as<uint32_t*>(), in_place ? td.as<const uint32_t*>() : ts.as<const uint32_t*>(), n_cols,
@@ -970,7 +969,8 @@ void evaluate_mixed(const uint32_t* const* src, const uint32_t* src_logs, uint32
     size_t n = kv.second.first.size();
     DevBuf ts = upload(kv.second.first.data(), n * sizeof(void*));
     DevBuf td = upload(kv.second.second.data(), n * sizeof(void*));
-    DevBuf ws = tile_workspace(false, use_matrices_evaluate(kv.first.first, kv.first.second, n), kv.first.second, tw, tree_len);
+    const uint32_t m = kv.first.second, blowup = m - kv.first.first;
+    DevBuf ws = tile_workspace(false, use_matrices_tile(m, n, false, blowup, false), m, tw, tree_len);
     evaluate_same_size(td.as<uint32_t*>(), ts.as<const uint32_t*>(), (uint32_t)n, kv.first.first, kv.first.second,
                        tw, tree_len, 0, ws.p, true);
   }

@@ -578,13 +578,6 @@ static void launch_contig(const uint32_t* const* src, uint32_t* const* dst, uint
   });
 }
 
-// From 2^24 values on: below, too few blocks have more than one column group to walk, and the
-// matrices' launch is not made up for (interpolation of 2^10: 2^13 columns 34.0 us against 38.7
-// here, 2^14 62.6 / 55.1, 2^16 174 / 155; evaluation on 2^12 from 2^10: 2^11 columns 43.4 / 48.8,
-// 2^12 of 2^12 67.4 / 65.1, 2^14 186 / 152).
-bool use_matrices_tile(uint32_t log_n, uint64_t n_cols) {
-  return log_n >= 10 && log_n <= 12 && (n_cols << log_n) >= (1ull << 24);
-}
 size_t tile_matrix_bytes(uint32_t log_n) { return (size_t)table_layout(log_n, log_n, 0).total * mm::MAT_BYTES; }
 void tile_matrices(bool inverse, uint32_t log_n, const uint32_t* tw, unsigned char* mats) {
   MatArgs A{};

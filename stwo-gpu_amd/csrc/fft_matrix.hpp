@@ -30,9 +30,29 @@ inline uint32_t groups_per_block(uint64_t n_groups, uint64_t tiles, uint32_t fil
   return (uint32_t)best;
 }
 
-// Whole small columns (log 10 .. 12), many at a time; mats: tile_matrix_bytes of device memory
-// filled by tile_matrices, tw / itw: the domain's tree part.
-bool use_matrices_tile(uint32_t log_n, uint64_t n_cols);
+// Whether a transform of n_cols whole columns over the domain of log_n (10 .. 12) runs on the matrix
+// cores; blowup (forward): log_n less the coefficients' log size.  The line lies where the pass has
+// made up for the launch that lays out its matrices (6 us), in millions (2^20) of values: 24 in place;
+// forward into other columns 32, 36, 48 and 80 (64 onto 2^10) at blowups 1, 2, 4 and 8, since the
+// butterflies skip the layers of the zero coefficients and the matrices do not; inverse into other
+// columns 36.  Matrix / butterfly time of a call just below and from the line on, for columns of 2^10,
+// 2^11 and 2^12:
+//   in place inverse      20: 1.05 1.02 0.99   24: 1.01 1.00 0.95   32: 0.97 0.97 0.92
+//   in place forward      20: 0.98 1.03 1.00   24: 0.95 0.99 0.96   32: 0.92 0.96 0.94
+//   forward, blowup 1     24: 1.01 1.03 1.02   32: 0.97 0.99 0.98   48: 0.95 0.98 0.95
+//   forward, blowup 2     32: 1.01 1.02 1.01   36: 0.99 0.94 0.97   48: 0.90 0.93 0.95
+//   forward, blowup 4     40: 1.00 1.02 1.01   48: 1.00 0.99 0.99   64: 0.88 0.96 0.94
+//   forward, blowup 8     64: 0.92 1.03 1.02   80: 0.90 0.98 0.96  128: 0.86 0.92 0.89
+//   inverse               32: 1.06 1.05 1.00   36: 1.00 0.98 0.95  128: 0.92 0.86 0.82
+inline bool use_matrices_tile(uint32_t log_n, uint64_t n_cols, bool inverse, uint32_t blowup, bool in_place) {
+  constexpr uint32_t FORWARD[4] = {32, 36, 48, 80};
+  if (log_n < 10 || log_n > 12 || blowup > 3) return false;
+  const uint64_t line = in_place && !blowup ? 24 : inverse ? 36 : blowup == 3 && log_n == 10 ? 64 : FORWARD[blowup];
+  return (n_cols << log_n) >= line << 20;
+}
+
+// The passes over whole small columns; mats: tile_matrix_bytes of device memory filled by
+// tile_matrices, tw / itw: the domain's tree part.
 size_t tile_matrix_bytes(uint32_t log_n);
 void tile_matrices(bool inverse, uint32_t log_n, const uint32_t* tw, unsigned char* mats);
 void interpolate_tiles(const uint32_t* const* src, uint32_t* const* dst, uint32_t n_cols, uint32_t log_n,

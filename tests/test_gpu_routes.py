@@ -1,0 +1,121 @@
+"""Which kernels a call runs, and its results at the sizes where that changes: the results of both forms
+are the same words, so the launches are counted too."""
+import contextlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+import oracle as O  # noqa: E402
+import stwo_hip as S  # noqa: E402
+
+
+@contextlib.contextmanager
+def launches(*names):
+    """Counts of the named launches inside the block, filled in at its end."""
+    got = {}
+    S.kernel_stats_reset()
+    S.kernel_timing(True)
+    try:
+        yield got
+        S.synchronize()
+        got.update({k: S.kernel_stats(k)[0] for k in names})
+    finally:
+        S.kernel_timing(False)
+
+
+def _filled(words, seed, column):
+    """A buffer of uniform values; the second column of `column` words holds the largest value throughout,
+    the last every other one."""
+    v = S.BaseFieldVec.uninitialized(words)
+    S.fill_uniform(v, seed)
+    most = np.full(column, S.P - 1, np.uint32)
+    S.check(S.lib().stwo_hip_memcpy(v.ptr + 4 * column, most.ctypes.data, 4 * column))
+    most[::2] = 0
+    S.check(S.lib().stwo_hip_memcpy(v.ptr + 4 * (words - column), most.ctypes.data, 4 * column))
+    return v
+
+
+def _part(v, first, n):
+    return S.BaseFieldVec.view(v.ptr + 4 * first, n).to_numpy()
+
+
+def _pointers(v, n_cols, words):
+    return S._ptr_array([v.ptr + 4 * words * c for c in range(n_cols)])
+
+
+# whole small columns: values from which the matrix cores take them, in millions (2^20)
+FORWARD = {(log, b): (32, 36, 48, 80)[b] for log in (10, 11, 12) for b in range(4)}
+FORWARD[10, 3] = 64
+
+
+@pytest.mark.parametrize("log_m,blowup", sorted(FORWARD))
+def test_evaluation_either_side_of_the_line(log_m, blowup):
+    """The fewest columns that take the matrix cores plus a remainder of a group, and one column less
+    than the line, into other columns."""
+    line = (FORWARD[log_m, blowup] << 20) >> log_m
+    log_n = log_m - blowup
+    coset = S.canonic_half_coset(log_m)
+    tw, _ = S.cached_twiddles(coset)
+    otw, _ = O.precompute_twiddles(coset.initial_index, coset.step_size, coset.log_size)
+    for n_cols, on_matrices in ((line + 1, 1), (line - 1, 0)):
+        src, dst = _filled(n_cols << log_n, 3 * log_m + blowup, 1 << log_n), S.BaseFieldVec.uninitialized(n_cols << log_m)
+        logs = np.full(n_cols, log_n, np.uint32), np.full(n_cols, log_m, np.uint32)
+        with launches("fft_matrices", "fft_fwd_tile") as got:
+            S.check(S.lib().stwo_hip_evaluate_columns_async(
+                _pointers(src, n_cols, 1 << log_n), logs[0].ctypes.data_as(S.u32p), _pointers(dst, n_cols, 1 << log_m),
+                logs[1].ctypes.data_as(S.u32p), n_cols, tw, 1 << coset.log_size))
+        assert got["fft_matrices"] == on_matrices
+        for c in (0, 1, n_cols // 2, n_cols - 2, n_cols - 1):
+            ext = np.zeros(1 << log_m, np.uint32)
+            ext[: 1 << log_n] = _part(src, c << log_n, 1 << log_n)
+            assert (_part(dst, c << log_m, 1 << log_m) == O.evaluate(ext, coset.initial_index, otw)).all(), c
+
+
+@pytest.mark.parametrize("log_n", [10, 11, 12])
+@pytest.mark.parametrize("in_place", [True, False])
+def test_interpolation_either_side_of_the_line(log_n, in_place):
+    line = ((24 if in_place else 36) << 20) >> log_n
+    coset = S.canonic_half_coset(log_n)
+    _, itw = S.cached_twiddles(coset)
+    _, oitw = O.precompute_twiddles(coset.initial_index, coset.step_size, coset.log_size)
+    for n_cols, on_matrices in ((line + 1, 1), (line - 1, 0)):
+        src = _filled(n_cols << log_n, log_n, 1 << log_n)
+        dst = src if in_place else S.BaseFieldVec.uninitialized(n_cols << log_n)
+        picks = (0, 1, n_cols // 2, n_cols - 2, n_cols - 1)
+        before = [_part(src, c << log_n, 1 << log_n) for c in picks]
+        logs = np.full(n_cols, log_n, np.uint32).ctypes.data_as(S.u32p)
+        sp, dp = _pointers(src, n_cols, 1 << log_n), _pointers(dst, n_cols, 1 << log_n)
+        with launches("fft_matrices") as got:
+            if in_place:
+                S.check(S.lib().stwo_hip_interpolate_columns_async(sp, logs, n_cols, itw, 1 << coset.log_size))
+            else:
+                S.check(S.lib().stwo_hip_interpolate_columns_oop_async(sp, dp, logs, n_cols, itw, 1 << coset.log_size))
+        assert got["fft_matrices"] == on_matrices
+        for c, v in zip(picks, before):
+            assert (_part(dst, c << log_n, 1 << log_n) == O.interpolate(v, coset.initial_index, oitw)).all(), c
+
+
+@pytest.mark.parametrize("log_n,blowup", [(10, 1), (11, 1), (12, 0), (9, 2)])
+def test_extension_of_small_columns(log_n, blowup):
+    """Extensions whose two halves take different forms: the inverse on butterflies, the forward half on
+    matrices or both on matrices."""
+    log_m = log_n + blowup
+    n_cols = max((FORWARD[log_m, blowup] << 20) >> log_m, 1) + 1
+    src, dst = _filled(n_cols << log_n, log_n, 1 << log_n), S.BaseFieldVec.uninitialized(n_cols << log_m)
+    picks = (0, n_cols // 2, n_cols - 1)
+    before = [_part(src, c << log_n, 1 << log_n) for c in picks]
+    coset = S.canonic_half_coset(log_m)
+    tw, itw = S.cached_twiddles(coset)
+    sp, dp = _pointers(src, n_cols, 1 << log_n), _pointers(dst, n_cols, 1 << log_m)
+    logs = np.full(n_cols, log_n, np.uint32).ctypes.data_as(S.u32p)
+    with launches("fft_matrices") as got:
+        S.check(S.lib().stwo_hip_lde_columns_async(sp, sp, dp, logs, n_cols, blowup, tw, itw, 1 << coset.log_size))
+    inverse = 10 <= log_n and (n_cols << log_n) >= 36 << 20
+    assert got["fft_matrices"] == 1 + inverse
+    otw, oitw = O.precompute_twiddles(coset.initial_index, coset.step_size, coset.log_size)
+    ocoef, olde = O.lde_columns(before, blowup, otw, oitw)
+    for i, c in enumerate(picks):
+        assert (_part(src, c << log_n, 1 << log_n) == ocoef[i]).all(), c
+        assert (_part(dst, c << log_m, 1 << log_m) == olde[i]).all(), c

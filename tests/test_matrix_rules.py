@@ -1,5 +1,5 @@
 """The host rules of the matrix-core FFT passes (stwo-gpu_amd/csrc/fft_matrix.hpp), built by the host
-compiler: how a pass is split into blocks."""
+compiler: how a pass is split into blocks, and which calls take the matrix cores."""
 import heapq
 import os
 import subprocess
@@ -71,3 +71,23 @@ def test_one_tile_beyond_the_caches(ask):
     for g in (8192, 16384, 1 << 18):
         (p,) = ask([("split", g, 1, 512)])
         assert -(-g // p) >= 4 * 512
+
+
+# calls timed with both forms in one process (median of 25, four times in turn): the matrices' time
+# over the butterflies', by log, values in millions (2^20) and kind
+BUTTERFLIES_FASTER = [(10, 16, 0), (10, 16, 2), (10, 16, 3), (10, 16, 8), (10, 20, 8), (11, 16, 0), (11, 16, 3), (11, 20, 1),
+                      (11, 20, 8), (11, 40, 3), (12, 16, 0), (12, 20, 2), (12, 24, 0), (12, 24, 8), (12, 28, 3), (12, 40, 3),
+                      (12, 52, 3), (11, 20, 24)]
+MATRICES_FASTER = [(10, 128, 0), (10, 64, 1), (10, 64, 2), (10, 64, 3), (10, 128, 8), (10, 32, 24), (10, 32, 16),
+                   (11, 48, 0), (11, 36, 1), (11, 64, 2), (11, 80, 3), (11, 96, 8), (11, 32, 24), (12, 40, 0), (12, 40, 1),
+                   (12, 64, 2), (12, 80, 3), (12, 36, 8), (12, 24, 24), (12, 32, 16)]
+
+
+def test_small_columns_take_the_faster_form(ask):
+    q = [("tile", log, (m << 20) >> log, kind) for log, m, kind in BUTTERFLIES_FASTER + MATRICES_FASTER]
+    assert ask(q) == [0] * len(BUTTERFLIES_FASTER) + [1] * len(MATRICES_FASTER)
+
+
+def test_small_columns_that_the_matrices_do_not_take(ask):
+    """Other sizes of domain, blowups above 8, and a source larger than the domain."""
+    assert ask([("tile", 9, 1 << 20, 0), ("tile", 13, 1 << 20, 0), ("tile", 12, 1 << 20, 4), ("tile", 12, 1 << 20, 7)]) == [0] * 4
