@@ -154,7 +154,7 @@ __device__ __forceinline__ qm31 combine(const Batch* __restrict__ batches, const
   return r;
 }
 
-// Column-major form for up to 4 batches and few samples (or more columns than MM_MAX_SLOTS): each
+// Column-major form for up to 4 batches and few samples (few_samples; or more columns than MM_MAX_SLOTS): each
 // sampled column value of a row is loaded once and multiplied into the sums of all NB batches,
 // with alpha = 0 for a batch that does not sample the column; loads run one group of QG columns
 // ahead of the arithmetic.  A batch's sums are folded after every fourth product taken into
@@ -255,12 +255,21 @@ constexpr uint32_t RING = DEPTH * KSTEP * 64, TILE = 256;  // words of a ring, o
 // Values from which the column reads are nontemporal (more than the caches hold: 200 columns of
 // 2^22, 1 point: 597 us instead of 634; below, 64 columns of 2^20: 84 us plain, 90 nontemporal).
 constexpr uint64_t MM_STREAM = 1ull << 27;
-// Samples from which the matrix form is taken, for one batch and for more.  Its weights are
-// expanded by a launch of their own instead of copied (3 us), and a batch alone fills half an
-// operand tile.  One point, cols / matrix: 96 columns of 2^20 93 / 102 us, 128 columns 120 / 112,
-// 64 of 2^12 18.7 / 21.9, 256 of 2^12 38 / 34.  Two to four points: 8 columns of 2^12, 2 points
-// 17.9 / 20.1 us, 32 columns 24.5 / 21.7; 32 columns of 2^20, 2 points 82 / 56.
-constexpr uint32_t FEW_ONE = 128, FEW = 32;
+// Whether a call samples so little that the multiply-adds are the faster form: the matrix form's
+// weights are expanded by a launch of their own instead of copied (3 us), and an odd batch fills half
+// an operand tile.  The more rows, the sooner that is made up; a batch's multiply-adds also run over
+// columns in groups of 16, sampled or not.  Matrix / multiply-add time of a call: one point, 112 samples
+// 0.93 .. 1.02 and 128 0.90 .. 1.01.  Two points, 16 columns at both up to 2^16 rows 1.04, 17 columns
+// 0.98, 16 of 2^17 1.00.  Three points, 16 columns at each up to 2^16 rows 1.07, 20 1.01, 24 1.00, 40
+// columns at one point each 0.98; 11 of 2^19 1.02, 14 1.00; 11 of 2^20 1.00.  Four points, 8 columns at
+// each up to 2^16 rows 1.03, 12 0.98, 32 columns at one point each 0.95; 8 of 2^17 0.97.
+inline bool few_samples(uint32_t n_batches, uint32_t log_size, uint64_t samples, uint32_t columns) {
+  if (samples < 32) return true;
+  if (n_batches == 1) return samples < 128;
+  if (n_batches == 2) return log_size < 17 && samples < 34;
+  if (n_batches == 3) return log_size < 19 ? samples < 64 && columns <= 32 : log_size == 19 && samples < 40;
+  return log_size < 17 && samples < 48 && columns <= 16;
+}
 constexpr uint32_t mm_tiles(uint32_t n_batches) { return (n_batches + 1) / 2; }
 constexpr uint32_t padded_slots(uint32_t n_cols) { return (n_cols + KSTEP - 1) / KSTEP * KSTEP; }
 
@@ -622,18 +631,11 @@ void launch_slots(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* c
         T, log_size, dsl, n_loop, dbs, out[0], out[1], out[2], out[3]);
   });
 }
-// column-major launch: per sampled column one slot with the alpha of every batch (0 when
-// the batch does not sample it; a column sampled twice in one batch gets the sum).  Returns
-// whether the columns are few enough for it.
+// matrix launch: slot_of[c] is the slot of sampled column c, n_used of them
 template <int NB>
-bool launch_matrix(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols, uint32_t n_cols,
-                    const std::vector<quot::Sample>& ss, const std::vector<quot::Batch>& bs, uint32_t* const out[4]) {
-  constexpr uint32_t NONE = ~0u;
-  std::vector<uint32_t> slot_of(n_cols, NONE);
-  uint32_t n_used = 0;
-  for (const quot::Sample& S : ss)
-    if (slot_of[S.col] == NONE) slot_of[S.col] = n_used++;
-  if (n_used > quot::MM_MAX_SLOTS) return false;
+void launch_matrix(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols,
+                   const std::vector<uint32_t>& slot_of, uint32_t n_used, const std::vector<quot::Sample>& ss,
+                   const std::vector<quot::Batch>& bs, uint32_t* const out[4]) {
   const uint32_t n_slots = quot::padded_slots(n_used);
   // host image: pointers | alphas | batches
   const size_t o_alpha = sizeof(void*) * n_slots, o_batch = o_alpha + sizeof(qm31) * NB * n_slots;
@@ -665,14 +667,20 @@ bool launch_matrix(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* 
                                                 (uint32_t*)(base + Y.weights), (uint32_t*)(base + Y.batches));
   });
   launch_mm<NB>(hi, hs, log_size, base, n_slots, out, 1, 0);
-  return true;
 }
 template <int NB>
 void launch_cols_nb(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols, uint32_t n_cols,
                     const std::vector<quot::Sample>& ss, const std::vector<quot::Batch>& bs, uint32_t* const out[4]) {
-  const bool few = ss.size() < (NB == 1 ? quot::FEW_ONE : quot::FEW);
-  if (few || !launch_matrix<NB>(hi, hs, log_size, h_cols, n_cols, ss, bs, out))
+  constexpr uint32_t NONE = ~0u;
+  std::vector<uint32_t> slot_of;
+  uint32_t n_used = 0;
+  if (ss.size() >= 32) slot_of.resize(n_cols, NONE);  // (fewer samples need no slots to decide)
+  for (const quot::Sample& S : ss)
+    if (!slot_of.empty() && slot_of[S.col] == NONE) slot_of[S.col] = n_used++;
+  if (n_used > quot::MM_MAX_SLOTS || quot::few_samples(NB, log_size, ss.size(), n_used))
     launch_slots<NB>(hi, hs, log_size, h_cols, ss, bs, out);
+  else
+    launch_matrix<NB>(hi, hs, log_size, h_cols, slot_of, n_used, ss, bs, out);
 }
 void launch_cols(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* const* h_cols, uint32_t n_cols,
                  const std::vector<quot::Sample>& ss, const std::vector<quot::Batch>& bs, uint32_t n_batches,

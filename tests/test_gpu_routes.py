@@ -119,3 +119,30 @@ def test_extension_of_small_columns(log_n, blowup):
     for i, c in enumerate(picks):
         assert (_part(src, c << log_n, 1 << log_n) == ocoef[i]).all(), c
         assert (_part(dst, c << log_m, 1 << log_m) == olde[i]).all(), c
+
+
+def _quotients(log_n, n_cols, n_points, dense):
+    """Quotients of n_cols columns sampled at every point or at one point each: launches that expand
+    weights, and whether the result is the oracle's."""
+    rng = np.random.default_rng(100 * log_n + n_cols)
+    host = [rng.integers(0, S.P, 1 << log_n, dtype=np.uint32) for _ in range(n_cols)]
+    host[0][:] = S.P - 1
+    cols = [S.BaseFieldVec.from_numpy(h) for h in host]
+    batches = [(S.random_circle_point_qm31(rng), [(c, S.random_qm31(rng)) for c in range(n_cols) if dense or c % n_points == k])
+               for k in range(n_points)]
+    rc, dom = S.random_qm31(rng), S.canonic_half_coset(log_n)
+    out = S.SecureColumn.uninitialized(1 << log_n)
+    with launches("quotient_constants") as got:
+        S.accumulate_quotients_async(dom, cols, rc, S.QuotientSamples(batches), out)
+    want = O.accumulate_quotients(dom.initial_index, dom.step_size, log_n, host, rc, batches)
+    assert (out.to_numpy() == want).all()
+    return got["quotient_constants"]
+
+
+# columns sampled at every point (or at one each): whether the matrix form is the faster one, as timed
+@pytest.mark.parametrize("log_n,n_cols,n_points,dense,matrix", [
+    (11, 112, 1, True, 0), (11, 128, 1, True, 1), (11, 16, 2, True, 0), (11, 17, 2, True, 1), (11, 16, 3, True, 0),
+    (11, 22, 3, True, 1), (11, 32, 3, False, 0), (11, 40, 3, False, 1), (11, 11, 4, True, 0), (11, 12, 4, True, 1),
+    (11, 32, 4, False, 1), (17, 16, 2, True, 1), (17, 8, 4, True, 1), (17, 16, 3, True, 0)])
+def test_quotients_take_the_faster_form(log_n, n_cols, n_points, dense, matrix):
+    assert _quotients(log_n, n_cols, n_points, dense) == matrix
