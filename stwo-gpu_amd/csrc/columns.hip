@@ -105,7 +105,7 @@ __device__ __forceinline__ uint32_t mirrored_order(uint32_t mid_bits) {
   return m;
 }
 
-// 4-byte elements in columns of at least 2^14: 128 x 128 tiles (512-byte runs), both tiles of the
+// 4-byte elements in columns of at least 2^14 (BR_BIG): 128 x 128 tiles (512-byte runs), both tiles of the
 // pair in registers and one padded LDS tile for the two transposes.  A wave's 16-byte accesses
 // cover two rows.  Bound by the memory system: 2^28 values 591 -> 499 us (4.3 TB/s), where the
 // same exchange of tiles without the transposes takes 460 and a pass over the tiles in place 390.
@@ -225,6 +225,12 @@ __global__ void bitrev_simple_kernel(T* a, uint32_t n, uint32_t log_n) {
 // column being larger than the caches.  Nontemporal / plain: 2^27 M31 253 / 280 us, 2^26 135 / 92;
 // 2^25 QM31 245 / 262, 2^24 138 / 95.
 constexpr uint32_t BR_STREAM = 27;
+// log of the 4-byte values from which 128 x 128 tiles fill the chip (256 blocks): below, a block that
+// turns a pair of them is the longer chain, and 32 x 32 tiles are faster.  Large / small tiles: 2^16
+// 15.7 / 14.2 us, 2^20 16.6 / 15.1, 2^21 17.1 / 16.3, 2^22 18.7 / 19.5, 2^24 34.9 / 39.9; columns off 16
+// bytes 2^20 17.2 / 15.5, 2^22 19.4 / 21.8.  In 2^14 and 2^15 values no large tile has a partner: 14.0 / 14.1
+// us, off 16 bytes 14.0 / 14.5.
+constexpr uint32_t BR_BIG = 22;
 template <class T>
 void bit_reverse(T* a, uint64_t n) {
   require(is_pow2(n) && n <= (1ull << 31), "bit_reverse: size must be a power of two <= 2^31");
@@ -233,7 +239,7 @@ void bit_reverse(T* a, uint64_t n) {
   if (log_n >= 2 * TA) {
     timed("bit_reverse", [&] {
       if constexpr (sizeof(T) == 4) {
-        if (log_n >= 14)
+        if (log_n >= BR_BIG || log_n == 14 || log_n == 15)
           (log_n >= BR_STREAM ? bitrev_big_kernel<true> : bitrev_big_kernel<false>)<<<1u << (log_n - 14), 512, 0,
                                                                                        ctx().cur>>>(a, log_n);
         else

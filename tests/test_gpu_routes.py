@@ -146,3 +146,17 @@ def _quotients(log_n, n_cols, n_points, dense):
     (11, 32, 4, False, 1), (17, 16, 2, True, 1), (17, 8, 4, True, 1), (17, 16, 3, True, 0)])
 def test_quotients_take_the_faster_form(log_n, n_cols, n_points, dense, matrix):
     assert _quotients(log_n, n_cols, n_points, dense) == matrix
+
+
+@pytest.mark.parametrize("log_n", [14, 15, 16, 21, 22])
+@pytest.mark.parametrize("offset", [0, 1, 2, 3])
+def test_bit_reverse_at_the_tile_sizes(log_n, offset):
+    """Columns at any word either side of the sizes at which the tile changes, nothing beyond their ends
+    touched."""
+    data = np.random.default_rng(log_n).integers(0, S.P, (1 << log_n) + 8, dtype=np.uint32)
+    col = S.BaseFieldVec.from_numpy(data)
+    S.lib().bit_reverse_base_field(col.ptr + 4 * offset, 1 << log_n)
+    S.check()
+    want = data.copy()
+    want[offset:offset + (1 << log_n)] = O.bit_reverse(data[offset:offset + (1 << log_n)].copy())
+    assert (col.to_numpy() == want).all()
