@@ -723,11 +723,11 @@ static void launch_pass(const PassPlan& p, const PassArgs& base) {
 
 // The matrices of a transform of whole small columns over the domain of log_n, when it uses them
 // (use_matrices_tile): enqueued before the pointer tables are uploaded, so they are made while the
-// host copies.
+// host copies, but allocated behind them: where memory holds the tables alone, butterflies take over.
 static DevBuf tile_workspace(bool inverse, bool used, uint32_t log_n, const uint32_t* tw, uint64_t tree_len) {
   if (!used || tree_len < (1ull << (log_n - 1))) return DevBuf();  // (a short tree is refused later)
-  DevBuf ws(tile_matrix_bytes(log_n));
-  tile_matrices(inverse, log_n, tw + (tree_len - (1ull << (log_n - 1))), ws.as<unsigned char>());
+  DevBuf ws = DevBuf::optional(tile_matrix_bytes(log_n));
+  if (ws.p) tile_matrices(inverse, log_n, tw + (tree_len - (1ull << (log_n - 1))), ws.as<unsigned char>());
   return ws;
 }
 
@@ -828,7 +828,7 @@ void lde_same_size(const uint32_t* const* d_src, uint32_t* const* d_coeffs, uint
   const uint32_t m = n + log_blowup;
   require(m <= 30, "lde: log size out of range");
   require(tree_len >= (1ull << (m - 1)), "lde: twiddle tree smaller than the evaluation domain");
-  if (var.mat && n >= 17 && n <= 20) {
+  if (var.mat && ws && n >= 17 && n <= 20) {
     lde_matrices(d_src, d_coeffs, d_lde, n_cols, n, log_blowup, tw + (tree_len - (1ull << (m - 1))),
                  itw + (tree_len - (1ull << (n - 1))), (unsigned char*)ws);
     return;
@@ -905,8 +905,7 @@ void lde_mixed(const uint32_t* const* src, uint32_t* const* coeffs, uint32_t* co
     DevBuf d = upload(t.data(), t.size() * sizeof(void*));
     const void* const* base = d.as<const void*>();
     const LdeVariant var = lde_variant_for(kv.first, log_blowup, cnt);
-    const size_t wb = lde_workspace_bytes(kv.first, log_blowup, cnt, var);
-    DevBuf ws = wb ? DevBuf(wb) : DevBuf();
+    const DevBuf ws = DevBuf::optional(lde_workspace_bytes(kv.first, log_blowup, cnt, var));
     lde_same_size((const uint32_t* const*)base, (uint32_t* const*)(base + cnt), (uint32_t* const*)(base + 2 * cnt),
                   (uint32_t)cnt, kv.first, log_blowup, tw, itw, tree_len, var, ws.p);
   }
@@ -917,9 +916,11 @@ void lde_mixed(const uint32_t* const* src, uint32_t* const* coeffs, uint32_t* co
 static void interpolate_one_size(uint32_t* const* cols, uint32_t n_cols, uint32_t log_n, const uint32_t* itw,
                                  uint64_t tree_len, const uint32_t* const* src) {
   const bool in_place = !src || std::equal(src, src + n_cols, (const uint32_t* const*)cols);
+  const size_t bytes = (size_t)n_cols * sizeof(void*);
+  DevBuf table(bytes), stable = src ? DevBuf(bytes) : DevBuf();
   DevBuf ws = tile_workspace(true, use_matrices_tile(log_n, n_cols, true, 0, in_place), log_n, itw, tree_len);
-  DevBuf table = upload(cols, (size_t)n_cols * sizeof(void*));
-  DevBuf stable = src ? upload(src, (size_t)n_cols * sizeof(void*)) : DevBuf();
+  upload_to(table.p, cols, bytes);
+  if (src) upload_to(stable.p, src, bytes);
   interpolate_same_size(table.as<uint32_t*>(), n_cols, log_n, itw, tree_len,
                         src ? stable.as<const uint32_t*>() : table.as<const uint32_t*>(), 0, ws.p, true);
 }
@@ -952,9 +953,11 @@ void evaluate_mixed(const uint32_t* const* src, const uint32_t* src_logs, uint32
       std::all_of(dst_logs, dst_logs + n_cols, [&](uint32_t l) { return l == dst_logs[0]; })) {
     const bool in_place = std::equal(src, src + n_cols, (const uint32_t* const*)dst);
     const uint32_t m = dst_logs[0], blowup = m - src_logs[0];
+    const size_t bytes = (size_t)n_cols * sizeof(void*);
+    DevBuf td(bytes), ts = in_place ? DevBuf() : DevBuf(bytes);
     DevBuf ws = tile_workspace(false, use_matrices_tile(m, n_cols, false, blowup, in_place), m, tw, tree_len);
-    DevBuf td = upload(dst, (size_t)n_cols * sizeof(void*));
-    DevBuf ts = in_place ? DevBuf() : upload(src, (size_t)n_cols * sizeof(void*));
+    upload_to(td.p, dst, bytes);
+    if (!in_place) upload_to(ts.p, src, bytes);
     evaluate_same_size(td.as<uint32_t*>(), in_place ? td.as<const uint32_t*>() : ts.as<const uint32_t*>(), n_cols,
                        src_logs[0], dst_logs[0], tw, tree_len, 0, ws.p, true);
     return;

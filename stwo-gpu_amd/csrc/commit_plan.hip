@@ -75,8 +75,8 @@ struct CommitPlan {
 
   void set_variant(Class& c, fft::LdeVariant v) const {
     c.var = v;
-    const size_t b = fft::lde_workspace_bytes(c.log, log_blowup, c.n, v);
-    c.ws = b ? DevBuf(b) : DevBuf();
+    c.ws = DevBuf();  // (given back before the next is taken)
+    c.ws = DevBuf::optional(fft::lde_workspace_bytes(c.log, log_blowup, c.n, v));
   }
 
   // Classes run on the auxiliary streams, largest first, round robin; each records an
@@ -157,6 +157,7 @@ struct CommitPlan {
       fft::LdeVariant best_v = cand[0];
       for (const auto& v : cand) {
         set_variant(c, v);
+        if (v.mat && !c.ws.p) continue;  // no memory for its matrices
         enqueue_class(c);  // warm-up
         float ms_min = 1e30f;
         for (int rep = 0; rep < 3; rep++) {
@@ -243,9 +244,7 @@ extern "C" int stwo_hip_commit_plan_create(StwoCommitPlan** out, uint32_t n_cols
         t[n + i] = coeffs[kv.second[i]];
         t[2 * n + i] = ldes[kv.second[i]];
       }
-      CommitPlan::Class c{kv.first, n, upload(t.data(), t.size() * sizeof(void*)), {}, DevBuf()};
-      p.set_variant(c, fft::lde_variant_for(kv.first, log_blowup, n));
-      p.classes.push_back(std::move(c));
+      p.classes.push_back(CommitPlan::Class{kv.first, n, upload(t.data(), t.size() * sizeof(void*)), {}, DevBuf()});
     }
     p.class_done.resize(p.classes.size());
     for (auto& e : p.class_done) hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
@@ -253,7 +252,13 @@ extern "C" int stwo_hip_commit_plan_create(StwoCommitPlan** out, uint32_t n_cols
     for (uint32_t i = 0; i < n_cols; i++) lde_logs[i] = log_sizes[i] + log_blowup;
     p.merkle = std::make_unique<merkle::MerklePlan>(n_cols, (const uint32_t* const*)ldes, lde_logs.data(),
                                                     (merkle::Hash* const*)layers, max_log);
-    if (autotune) {
+    // behind everything that the plan cannot do without, so that they take what memory is left
+    auto set_variants = [&] {
+      for (CommitPlan::Class& c : p.classes) p.set_variant(c, fft::lde_variant_for(c.log, log_blowup, c.n));
+    };
+    if (!autotune) {
+      set_variants();
+    } else {
       // the autotuner runs the plan several times on the caller's buffers; a column whose
       // coefficients alias its evaluations is interpolated in place by every run, so its
       // evaluations are kept aside and put back before create returns
@@ -270,6 +275,7 @@ extern "C" int stwo_hip_commit_plan_create(StwoCommitPlan** out, uint32_t n_cols
         hip_check(hipMemcpyAsync(sv.copy.p, sv.col, bytes, hipMemcpyDeviceToDevice, ctx().cur), "hipMemcpyAsync D2D");
         saved.push_back(std::move(sv));
       }
+      set_variants();
       p.autotune();
       for (Saved& sv : saved)
         hip_check(hipMemcpyAsync(sv.col, sv.copy.p, sv.bytes, hipMemcpyDeviceToDevice, ctx().cur),

@@ -17,12 +17,13 @@ struct LdeVariant {
 };
 
 // Device memory that lde_same_size needs beside the columns for this shape and variant
-// (matrices of the matrix-core passes; 0: none).
+// (matrices of the matrix-core passes; 0: none).  Without it the passes run on butterflies: callers
+// take it as DevBuf::optional, so no call needs more memory than its columns and tables.
 size_t lde_workspace_bytes(uint32_t n, uint32_t log_blowup, uint64_t n_cols, LdeVariant var);
 
 // Interpolate d_src into d_coeffs (may alias) and evaluate on the canonic domain of log
 // n + log_blowup into d_lde; device pointer tables of n_cols columns; allocates nothing.
-// ws: lde_workspace_bytes of device memory, written by each call.
+// ws: lde_workspace_bytes of device memory, written by each call; null: the butterfly passes of var.
 void lde_same_size(const uint32_t* const* d_src, uint32_t* const* d_coeffs, uint32_t* const* d_lde, uint32_t n_cols,
                    uint32_t n, uint32_t log_blowup, const uint32_t* tw, const uint32_t* itw, uint64_t tree_len,
                    LdeVariant var, void* ws);

@@ -425,10 +425,6 @@ Job::Job(const Params& p_, hipStream_t s, uint32_t n_jobs_)
   Arena A(p, L);
   jstride = n_jobs > 1 ? job_stride(p, L) : 0;
   arena = DevBuf(n_jobs > 1 ? jstride * n_jobs : A.end);
-  const LdePlans lde_plans(p, n_jobs);
-  var_t = lde_plans.t;
-  var_q = lde_plans.q;
-  if (lde_plans.ws) fft_ws = DevBuf(lde_plans.ws);
   char* base = arena.as<char>();
   coeffs = (uint32_t*)(base + A.coeffs);
   lde = (uint32_t*)(base + A.lde);
@@ -479,6 +475,10 @@ Job::Job(const Params& p_, hipStream_t s, uint32_t n_jobs_)
   const uint64_t o_ops = tb_bytes;
   tb_bytes += align256(sizeof(GatherOp) * gather_ops_upper_bound(p, L));
   tables_ = DevBuf(tb_bytes);
+  const LdePlans lde_plans(p, n_jobs);
+  var_t = lde_plans.t;
+  var_q = lde_plans.q;
+  fft_ws = DevBuf::optional(lde_plans.ws);  // (behind the buffers that the job cannot do without)
   char* dtab = tables_.as<char>();
   std::vector<char> image(tb_bytes);
   memcpy(image.data(), t.data(), t.size() * sizeof(void*));

@@ -48,7 +48,7 @@ struct Job {
   uint64_t jstride;
   DevBuf arena;  // every per-job device buffer, n_jobs arenas of jstride bytes
   fft::LdeVariant var_t, var_q;  // schedules of the trace's and the composition's extension
-  DevBuf fft_ws;                 // their workspace, one after the other
+  DevBuf fft_ws;                 // their workspace, one after the other (empty: butterflies)
   std::unique_ptr<merkle::MerklePlan> tree_t, tree_q;
   std::vector<std::unique_ptr<merkle::MerklePlan>> tree_l;
   DevBuf tables_;  // pointer tables, Merkle plan tables and the gather table

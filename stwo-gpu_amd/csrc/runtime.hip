@@ -134,6 +134,11 @@ size_t Pool::round(size_t b) {
   return (b + (2u << 20) - 1) & ~(size_t)((2u << 20) - 1);
 }
 void* Pool::alloc(size_t bytes) {
+  void* p = try_alloc(bytes);
+  if (!p) fail(STWO_HIP_ERR_NOMEM, "hipMalloc(%zu bytes) failed: %s", round(bytes), hipGetErrorString(hipErrorOutOfMemory));
+  return p;
+}
+void* Pool::try_alloc(size_t bytes) {
   size_t r = round(bytes);
   const hipStream_t cur = g_ctx.cur;
   for (auto it = cache_.lower_bound(r); it != cache_.end() && it->first <= r + r / 4; ++it) {  // close fit only
@@ -154,7 +159,8 @@ void* Pool::alloc(size_t bytes) {
     e = hipMalloc(&p, r);
     if (e != hipSuccess) {
       (void)hipGetLastError();
-      fail(STWO_HIP_ERR_NOMEM, "hipMalloc(%zu bytes) failed: %s", r, hipGetErrorString(e));
+      if (e != hipErrorOutOfMemory) fail(STWO_HIP_ERR_NOMEM, "hipMalloc(%zu bytes) failed: %s", r, hipGetErrorString(e));
+      return nullptr;
     }
   }
   live_[p] = r;

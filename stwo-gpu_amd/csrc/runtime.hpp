@@ -38,6 +38,7 @@ inline void require(bool ok, const char* fmt, const char* detail = "") {
 class Pool {
  public:
   void* alloc(size_t bytes);  // for work launched on ctx().cur
+  void* try_alloc(size_t bytes);  // the same, null where device memory does not hold it
   void free(void* p);         // every user of p is already enqueued on ctx().cur
   void release_cached();      // synchronises the device, then returns cached blocks to HIP
   size_t cached_bytes() const { return cached_; }
@@ -118,6 +119,12 @@ struct DevBuf {
   void* p = nullptr;
   DevBuf() = default;
   explicit DevBuf(size_t bytes) { p = ctx().pool.alloc(bytes); }
+  // a buffer that work gets faster by but not right: empty where device memory does not hold it
+  static DevBuf optional(size_t bytes) {
+    DevBuf b;
+    if (bytes) b.p = ctx().pool.try_alloc(bytes);
+    return b;
+  }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
   DevBuf(DevBuf&& o) noexcept : p(o.p) { o.p = nullptr; }
