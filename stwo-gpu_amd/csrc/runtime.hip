@@ -279,19 +279,25 @@ static bool device_to_host(const void* dst, const void* src, size_t bytes) {
   if (!ok) (void)hipGetLastError();  // (a pointer that the runtime does not know is no error here)
   return ok;
 }
+// waits for the stream that the copy below is on
+static void sync_current() {
+  if (g_ctx.cur == g_ctx.stream)
+    sync();
+  else
+    hip_check(hipStreamSynchronize(g_ctx.cur), "hipStreamSynchronize");
+}
 void download(void* host, const void* dev, size_t bytes) {
   if (!bytes) return;
-  if (bytes > DOWNLOAD_KERNEL_MAX || bytes % 4 || (uintptr_t)dev % 4 || g_ctx.cur != g_ctx.stream ||
-      !device_to_host(host, dev, bytes)) {
+  if (bytes > DOWNLOAD_KERNEL_MAX || bytes % 4 || (uintptr_t)dev % 4 || !device_to_host(host, dev, bytes)) {
     hip_check(hipMemcpyAsync(host, dev, bytes, hipMemcpyDefault, g_ctx.cur), "hipMemcpy");
-    sync();
+    sync_current();
     return;
   }
   Staging& st = take_staging(bytes);
   const uint32_t n4 = (uint32_t)(bytes / 4);
   download_kernel<<<(n4 + 255) / 256, 256, 0, g_ctx.cur>>>((uint32_t*)st.host, (const uint32_t*)dev, n4);
   hip_check(hipGetLastError(), "download_kernel");
-  sync();
+  sync_current();
   memcpy(host, st.host, bytes);  // (the buffer is free again: nothing else was taken meanwhile)
 }
 

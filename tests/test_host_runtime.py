@@ -29,6 +29,25 @@ def memory_limit(tmp_path_factory):
     return run
 
 
+@pytest.fixture(scope="module")
+def downloads(tmp_path_factory):
+    hipcc = os.environ.get("HIPCC", os.path.join(ROCM, "bin", "hipcc"))
+    if not os.path.exists(hipcc):
+        pytest.skip("hipcc not found")
+    out = str(tmp_path_factory.mktemp("download") / "download_check")
+    subprocess.run([hipcc, "-x", "hip", "--offload-arch=gfx950", "-std=c++17", "-O1", "-I" + os.path.join(ROOT, "include"),
+                    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                    os.path.join(HERE, "download_check.cpp"), "-o", out], check=True, capture_output=True)
+    return subprocess.run([out], capture_output=True, text=True, check=True).stdout.splitlines()
+
+
+@pytest.mark.parametrize("stream", [0, 1], ids=["library stream", "another current stream"])
+def test_copies_are_complete_on_return(downloads, stream):
+    """Small and large copies to host memory, one on the device, one of odd length: each is enqueued on the
+    current stream, and that stream is waited for."""
+    assert downloads[stream].split() == ["11"] * 4
+
+
 MIB = 1024
 
 
