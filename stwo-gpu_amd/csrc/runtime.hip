@@ -359,6 +359,7 @@ extern "C" int stwo_hip_free(void* ptr) {
 }
 extern "C" int stwo_hip_memcpy(void* dst, const void* src, size_t bytes) {
   return guarded([&] {
+    if (!bytes) return sync();  // synchronous with the library's work also where there is nothing to copy
     download(dst, src, bytes);
   });
 }

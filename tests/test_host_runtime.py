@@ -48,6 +48,10 @@ def test_copies_are_complete_on_return(downloads, stream):
     assert downloads[stream].split() == ["11"] * 4
 
 
+def test_copy_of_nothing_waits(downloads):
+    assert downloads[2] == "1"
+
+
 MIB = 1024
 
 
