@@ -281,7 +281,7 @@ __host__ __device__ __forceinline__ uint32_t weight_word(uint32_t slot, uint32_t
   return ((slot / KSTEP * tiles + batch / 2) * 64 + ((slot >> 2) & 1) * 32 + (batch & 1) * 16) * 4 + (slot & 3);
 }
 
-// From a host image (pinned memory or an upload) to the kernel's tables: column pointers and
+// From a host image (pinned memory) to the kernel's tables: column pointers and
 // batches copied, alphas ([slot][batch], n_slots x n_batches) expanded to weights.
 __global__ __launch_bounds__(256) void weights_kernel(const uint2* __restrict__ ptrs, const qm31* __restrict__ alphas,
                                                       const uint32_t* __restrict__ batch_words, uint32_t n_slots,
@@ -643,9 +643,10 @@ void launch_matrix(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* 
   // host image: pointers | alphas | batches
   const size_t o_alpha = sizeof(void*) * n_slots, o_batch = o_alpha + sizeof(qm31) * NB * n_slots;
   const size_t bytes = o_batch + sizeof(quot::Batch) * NB;
-  std::vector<unsigned char> big(bytes > HOST_BLOCK_MAX ? bytes : 0);
-  HostBlock pinned(big.empty() ? bytes : 16);
-  unsigned char* const host = big.empty() ? pinned.as<unsigned char>() : big.data();
+  static_assert((sizeof(void*) + sizeof(qm31) * NB) * quot::MM_MAX_SLOTS + sizeof(quot::Batch) * NB <= HOST_BLOCK_MAX,
+                "the largest image fits pinned memory");
+  HostBlock pinned(bytes);
+  unsigned char* const host = pinned.as<unsigned char>();
   memset(host, 0, bytes);
   const uint32_t** ptrs = (const uint32_t**)host;
   qm31* alphas = (qm31*)(host + o_alpha);
@@ -658,16 +659,14 @@ void launch_matrix(uint32_t hi, uint32_t hs, uint32_t log_size, const uint32_t* 
     }
   for (uint32_t i = n_used; i < n_slots; i++) ptrs[i] = ptrs[0];
   memcpy(host + o_batch, bs.data(), sizeof(quot::Batch) * NB);
-  const DevBuf up = big.empty() ? DevBuf() : upload(host, bytes);
-  const unsigned char* const src = big.empty() ? host : up.as<unsigned char>();
   const MmLayout Y(n_slots, NB);
   DevBuf d(Y.end);
   char* const base = d.as<char>();
   timed("quotient_constants", [&] {
     const uint32_t threads = std::max<uint32_t>(n_slots * 2 * quot::mm_tiles(NB), NB * sizeof(quot::Batch) / 4);
-    quot::weights_kernel<<<ceil_div(threads, 256), 256, 0, ctx().cur>>>((const uint2*)src, (const qm31*)(src + o_alpha),
-                                                (const uint32_t*)(src + o_batch), n_slots, NB, (uint2*)base,
-                                                (uint32_t*)(base + Y.weights), (uint32_t*)(base + Y.batches));
+    quot::weights_kernel<<<ceil_div(threads, 256), 256, 0, ctx().cur>>>(
+        (const uint2*)host, (const qm31*)(host + o_alpha), (const uint32_t*)(host + o_batch), n_slots, NB, (uint2*)base,
+        (uint32_t*)(base + Y.weights), (uint32_t*)(base + Y.batches));
   });
   launch_mm<NB>(hi, hs, log_size, base, n_slots, out, 1, 0);
 }
