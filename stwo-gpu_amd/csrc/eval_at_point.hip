@@ -89,27 +89,25 @@ __global__ void factors_kernel(const qm31* __restrict__ point, uint32_t L, Facto
   point_factors(point[0], point[1], L, *jptr(F, jo));
 }
 
-// block (b, col) folds coefficients [b 2^cb, (b+1) 2^cb) of column col
-__global__ __launch_bounds__(NT) void first_pass_cols(const uint32_t* const* __restrict__ cols, uint32_t L,
-                                                      uint32_t cb, const Factors* __restrict__ F, qm31* partial,
-                                                      uint64_t js) {
+// a whole column of at most 2^CB coefficients per block (blockIdx.y)
+__global__ __launch_bounds__(NT) void fold_cols(const uint32_t* const* __restrict__ cols, uint32_t L,
+                                                const Factors* __restrict__ F, qm31* out, uint64_t js) {
   __shared__ qm31 s[1 << (CB - 1)];
   const uint64_t jo = job_offset(js);
   F = jptr(F, jo);
-  partial = jptr(partial, jo);
+  out = jptr(out, jo);
   const uint32_t* c = jptr(cols[blockIdx.y], jo);
-  const uint32_t pairs = 1u << (cb - 1);
-  const size_t base = (size_t)blockIdx.x << cb;
+  const uint32_t pairs = 1u << (L - 1);
   const qm31 fy = F->f[L - 1];
   for (uint32_t i = threadIdx.x; i < pairs; i += NT) {
-    uint32_t c0 = c[base + 2 * i], c1 = c[base + 2 * i + 1];
+    uint32_t c0 = c[2 * i], c1 = c[2 * i + 1];
     qm31 v = qscale(fy, c1);
     v.x.a = add(v.x.a, c0);
     s[i] = v;
   }
   __syncthreads();
   tree_reduce(s, pairs, *F, (int)L - 2);
-  if (threadIdx.x == 0) partial[(size_t)blockIdx.y * gridDim.x + blockIdx.x] = s[0];
+  if (threadIdx.x == 0) out[blockIdx.y] = s[0];
 }
 
 // ---- columns of log >= 12 as a product with a basis on the matrix cores ------------------
@@ -272,20 +270,6 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const qm31* __restric
   if (t == 0) out[c] = qadd(qadd(ws[0], ws[1]), qadd(ws[2], ws[3]));
 }
 
-__global__ __launch_bounds__(NT) void reduce_pass_dev(const qm31* in, uint32_t g, const Factors* __restrict__ F,
-                                                      int fi, qm31* out, uint64_t js) {
-  __shared__ qm31 s[1 << (CB - 1)];
-  const uint64_t jo = job_offset(js);
-  in = jptr(in, jo);
-  F = jptr(F, jo);
-  out = jptr(out, jo);
-  const uint32_t cnt = 1u << g;
-  for (uint32_t i = threadIdx.x; i < cnt; i += NT) s[i] = in[((size_t)blockIdx.x << g) + i];
-  __syncthreads();
-  tree_reduce(s, cnt, *F, fi);
-  if (threadIdx.x == 0) out[blockIdx.x] = s[0];
-}
-
 }  // namespace eap
 
 // Columns of log >= 12: factors of two points | Lo | Mid operands | Hi | partial sums.  The bound
@@ -293,8 +277,7 @@ __global__ __launch_bounds__(NT) void reduce_pass_dev(const qm31* in, uint32_t g
 // callers' limits it sets; gemv_layout stays within it.
 size_t eval_at_point_columns_scratch_bytes(uint32_t n_cols, uint32_t L) {
   if (L >= eap::MIN_GEMV_LOG) return 512 + sizeof(qm31) * (4096 + (1ull << (L - 12)) * (1 + (size_t)n_cols));
-  const uint32_t cb = std::min<uint32_t>(L, eap::CB);
-  return 512 + 2 * sizeof(qm31) * (size_t)n_cols * (1ull << (L - cb));
+  return 512 + 2 * sizeof(qm31) * (size_t)n_cols;  // (the factors take 496; callers' limits are set by this)
 }
 
 namespace {
@@ -317,29 +300,12 @@ struct GemvLayout {
 static void eval_at_point_small_columns_async(const uint32_t* const* d_cols, uint32_t n_cols, uint32_t L,
                                               const qm31* d_point, qm31* d_out, void* d_scratch, uint32_t n_jobs,
                                               uint64_t js) {
+  static_assert(eap::MIN_GEMV_LOG == eap::CB + 1, "a small column is one block");
   eap::Factors* F = (eap::Factors*)d_scratch;
-  // small columns (log < 12): fold in LDS, block results reduced by later passes
-  const uint32_t cb = std::min<uint32_t>(L, eap::CB);
-  uint32_t blocks = 1u << (L - cb);
-  qm31* pa = (qm31*)((char*)d_scratch + 512);
-  qm31* pb = pa + (size_t)n_cols * blocks;
   timed("eval_at_point", [&] {
     eap::factors_kernel<<<dim3(1, 1, n_jobs), 1, 0, ctx().cur>>>(d_point, L, F, js);
-    eap::first_pass_cols<<<dim3(blocks, n_cols, n_jobs), eap::NT, 0, ctx().cur>>>(d_cols, L, cb, F,
-                                                                                   blocks == 1 ? d_out : pa, js);
+    eap::fold_cols<<<dim3(1, n_cols, n_jobs), eap::NT, 0, ctx().cur>>>(d_cols, L, F, d_out, js);
   });
-  int fi = (int)(L - cb) - 1;
-  while (blocks > 1) {
-    const uint32_t g = std::min<uint32_t>(log2_exact(blocks), eap::CB - 1);
-    const uint32_t nb = blocks >> g;
-    qm31* dst = nb == 1 ? d_out : pb;
-    timed("eval_at_point", [&] {
-      eap::reduce_pass_dev<<<dim3(nb * n_cols, 1, n_jobs), eap::NT, 0, ctx().cur>>>(pa, g, F, fi, dst, js);
-    });
-    std::swap(pa, pb);
-    fi -= (int)g;
-    blocks = nb;
-  }
 }
 
 // d_out[k n_cols + c] = value at point k, d_points[2k], d_points[2k + 1] = (x, y), of the polynomial
