@@ -17,15 +17,15 @@ namespace tw {
 
 // Level 0 holds the x of initial + step * brev(i): bit b of i contributes the fixed point
 // weight[b] = step * 2^(half_log - 1 - b), so a thread multiplies the weights of its set bits
-// and then takes its 16 values from one product each with 16 uniform points.  The level above
+// and then takes its 4 or 16 values from one product each with as many uniform points.  The level above
 // needs no points: brev(2i) over one more bit is brev(i), so entry i of level j + 1 is the
-// doubling x -> 2x^2 - 1 of entry 2i of level j, and a block that owns 2^12 consecutive values
-// of level 0 owns 2^11 of level 1, ... , one of level 12, and, where its index is a multiple of
-// 2^z, one of levels 12 + 1 .. 12 + z.  Bound by the latency of the products and of the
+// doubling x -> 2x^2 - 1 of entry 2i of level j, and a block that owns 2^B consecutive values
+// (B = 10 or 12) of level 0 owns 2^(B-1) of level 1, ... , one of level B, and, where its index is a
+// multiple of 2^z, one of levels B + 1 .. B + z.  Bound by the latency of the products and of the
 // doublings (2^22: 103 -> 13.8 us against a full power of the step per entry, which took 2 x 31
 // products each; the stores alone take 3 us).
 constexpr uint32_t TREE_NT = 256;
-// Blocks of 2^12 values, or of 2^10: a quarter of the chain of products and doublings and four times
+// Blocks of 2^12 values (trees from 2^21 on fill their four groups of 2^10), or of 2^10: a quarter of the chain of products and doublings and four times
 // the blocks, for trees up to 2^20 (a call with the inverses: 2^14 25.2 us with the small blocks, 28.3
 // with the large; 2^20 28.5 / 31.2; 2^21 33.6 / 33.4; 2^22 43.6 / 39.5; a power per entry took 25.4,
 // 46, 70 and 120).
@@ -51,21 +51,18 @@ __global__ __launch_bounds__(TREE_NT) void tree_kernel(uint32_t* __restrict__ ou
     const pt r = pmul(q, A.weight[b + 2]);
     if ((t >> b) & 1) q = r;
   }
-  // value c of group k: index i = blk 2^12 + 2^10 k + 4 t + c (a small tree has fewer groups)
+  // value c of group k: index i = blk 2^BLOCK_LOG + 2^10 k + 4 t + c (blocks of several groups are for
+  // trees that fill them; of a single group that is more than the tree, values past half are not stored)
   constexpr int GROUPS = 1 << (BLOCK_LOG - 10);
-  const uint32_t groups = min((uint32_t)GROUPS, (half + 1023) >> 10);
   uint32_t x[GROUPS][4];
 #pragma unroll
-  for (int k = 0; k < GROUPS; k++) {
-    if (k >= (int)groups) break;  // uniform, here and below
+  for (int k = 0; k < GROUPS; k++)
 #pragma unroll
     for (int c = 0; c < 4; c++) x[k][c] = pmul(q, A.lane16[4 * k + c]).x;
-  }
   auto twice = [](uint32_t v) { return sub(canon(2 * sqr(v)), 1); };
   // level j starts at size - (size >> j); j <= 2: 4, 2, 1 values per thread and group
 #pragma unroll
   for (int k = 0; k < GROUPS; k++) {
-    if (k >= (int)groups) break;
     const uint32_t i = (blk << BLOCK_LOG) + (k << 10) + 4 * t;
 #pragma unroll
     for (int j = 0; j < 3; j++) {
@@ -84,7 +81,6 @@ __global__ __launch_bounds__(TREE_NT) void tree_kernel(uint32_t* __restrict__ ou
     uint32_t* lvl = out + (size - (size >> j));
 #pragma unroll
     for (int k = 0; k < GROUPS; k++) {
-      if (k >= (int)groups) break;
       const uint32_t i = (blk << BLOCK_LOG) + (k << 10) + 4 * t;
       if ((t & ((1u << (j - 2)) - 1)) == 0 && i < half) lvl[i >> j] = x[k][0];
       x[k][0] = twice(x[k][0]);
@@ -97,7 +93,6 @@ __global__ __launch_bounds__(TREE_NT) void tree_kernel(uint32_t* __restrict__ ou
     uint32_t* lvl = out + (size - (size >> j));
 #pragma unroll
     for (int k = 0; k < GROUPS; k++) {
-      if (k >= (int)groups) break;
       const uint32_t i = (blk << BLOCK_LOG) + (k << 10);
       if ((i & ((1u << j) - 1)) == 0 && i < half) lvl[i >> j] = x[k][0];
       x[k][0] = twice(x[k][0]);
