@@ -224,3 +224,26 @@ def mle_eval(evals, r):
         fx = f if isinstance(f, tuple) else qm(int(f))
         total = qm_add(total, qm_mul(fx, eq_poly(index_bits(x, n), r)))
     return total
+
+
+# ---- one row of the DEEP quotients (quotients.cu:111-178) ----
+def quotient_at_row(half_coset, log_size, row, values, random_coeff, batches):
+    """The accumulated quotient at a row of the bit-reversed domain of 2^log_size points over
+    half_coset; values[c]: column c at that row; batches: [(point, [(column, value), ...]), ...]."""
+    i, half = brev(row, log_size), 1 << (log_size - 1)
+    x, y = point_at_index(half_coset.initial_index + half_coset.step_size * (i % half))
+    if i >= half:
+        y = (P - y) % P
+    acc = qm(0)
+    for (px, py), samples in batches:
+        c = qm_sub(qm_conj(py), py)
+        alpha, num = qm(1), qm(0)
+        for column, v in samples:
+            alpha = qm_mul(alpha, random_coeff)
+            a = qm_sub(qm_conj(v), v)
+            b = qm_sub(qm_mul(v, c), qm_mul(a, py))
+            num = qm_add(num, qm_mul(alpha, qm_sub(qm_scale(c, values[column]), qm_add(qm_scale(a, y), b))))
+        den = qm_sub(qm_mul(qm_sub(px[:2] + (0, 0), qm(x)), py[2:] + (0, 0)),
+                     qm_mul(qm_sub(py[:2] + (0, 0), qm(y)), px[2:] + (0, 0)))
+        acc = qm_add(qm_mul(acc, qm_pow(random_coeff, len(samples))), qm_div(num, den))
+    return acc

@@ -8,6 +8,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 import oracle as O  # noqa: E402
+import refmath as R  # noqa: E402
 import stwo_hip as S  # noqa: E402
 
 
@@ -160,3 +161,55 @@ def test_bit_reverse_at_the_tile_sizes(log_n, offset):
     want = data.copy()
     want[offset:offset + (1 << log_n)] = O.bit_reverse(data[offset:offset + (1 << log_n)].copy())
     assert (col.to_numpy() == want).all()
+
+
+@pytest.mark.parametrize("log_n,n_cols,blowup", [
+    (17, 385, 1), (17, 1024, 1), (17, 1024, 2), (17, 390, 4), (18, 200, 1), (18, 513, 2), (19, 101, 1), (19, 256, 2), (19, 97, 3),
+    (20, 67, 1), (20, 128, 1), (20, 128, 2), (20, 72, 3)])
+def test_extension_passes(log_n, n_cols, blowup):
+    """Every number of strided layers on the matrix cores, two and more blocks of the evaluation domain,
+    below and above the size from which accesses stream (2^27 values), uneven groups of columns."""
+    log_m = log_n + blowup
+    src, dst = _filled(n_cols << log_n, log_n + n_cols, 1 << log_n), S.BaseFieldVec.uninitialized(n_cols << log_m)
+    picks = (0, 1, n_cols // 2, n_cols - 1)
+    before = [_part(src, c << log_n, 1 << log_n) for c in picks]
+    coset = S.canonic_half_coset(log_m)
+    tw, itw = S.cached_twiddles(coset)
+    sp, dp = _pointers(src, n_cols, 1 << log_n), _pointers(dst, n_cols, 1 << log_m)
+    logs = np.full(n_cols, log_n, np.uint32).ctypes.data_as(S.u32p)
+    with launches("fft_matrices", "fft_lde_strided") as got:
+        S.check(S.lib().stwo_hip_lde_columns_async(sp, sp, dp, logs, n_cols, blowup, tw, itw, 1 << coset.log_size))
+    assert got == {"fft_matrices": 1, "fft_lde_strided": 1}
+    otw, oitw = O.precompute_twiddles(coset.initial_index, coset.step_size, coset.log_size)
+    ocoef, olde = O.lde_columns(before, blowup, otw, oitw)
+    for i, c in enumerate(picks):
+        assert (_part(src, c << log_n, 1 << log_n) == ocoef[i]).all(), c
+        assert (_part(dst, c << log_m, 1 << log_m) == olde[i]).all(), c
+
+
+@pytest.mark.parametrize("log_n,n_cols,n_points", [(20, 128, 1), (20, 131, 2), (20, 129, 3), (21, 64, 4), (21, 72, 2)])
+def test_quotients_of_streamed_columns(log_n, n_cols, n_points):
+    """The matrix form with one to four points where the columns are read past the caches; rows at the
+    domain's ends and inside against the formula."""
+    src = _filled(n_cols << log_n, n_cols, 1 << log_n)
+    cols = [S.BaseFieldVec.view(src.ptr + (c << (log_n + 2)), 1 << log_n) for c in range(n_cols)]
+    rng = np.random.default_rng(n_cols)
+    batches = [(S.random_circle_point_qm31(rng), [(c, S.random_qm31(rng)) for c in range(n_cols) if n_points == 1 or (c + k) % 3])
+               for k in range(n_points)]
+    rc, dom = S.random_qm31(rng), S.canonic_half_coset(log_n)
+    out = S.SecureColumn.uninitialized(1 << log_n)
+    with launches("quotient_constants") as got:
+        S.accumulate_quotients_async(dom, cols, rc, S.QuotientSamples(batches), out)
+    assert got["quotient_constants"] == 1
+    result = out.to_numpy()
+    rows = [0, 1, 63, 64, 511, 512, (1 << log_n) // 3, (1 << log_n) - 2, (1 << log_n) - 1]
+    values = {c: [int(_part(col, r, 1)[0]) for r in rows] for c, col in enumerate(cols)}
+    for i, r in enumerate(rows):
+        want = R.quotient_at_row(dom, log_n, r, {c: v[i] for c, v in values.items()}, rc, batches)
+        assert tuple(int(result[k][r]) for k in range(4)) == want, r
+
+
+@pytest.mark.parametrize("n_cols,matrix", [(8192, 1), (8193, 0)])
+def test_quotients_at_the_most_columns(n_cols, matrix):
+    """The matrix form's sums are bounded for 8192 columns; one more takes the other form."""
+    assert _quotients(4, n_cols, 1, True) == matrix
