@@ -177,7 +177,8 @@ def bench_lde_commit(args):
         "data": "synthetic (uniform M31, seeded counter-based stream)",
         "config": {"workload": "LDE+commit: 256 M31 columns log 20 -> LDE log 21 (blowup 2) + Blake2s Merkle",
                    "columns": C, "log_size": LOG_N, "log_blowup": LOG_BLOWUP, "parallelism": "single GPU",
-                   "fft_schedule": {"contiguous_layers": schedule[0], "fused_strided": schedule[1]},
+                   "fft_schedule": {"contiguous_layers": schedule[0], "fused_strided": schedule[1],
+                                    "matrix_cores": bool(stats["fft_matrices"][0])},
                    "launch": ("hipGraph replay of the commit plan" if plan.uses_graph() else
                               "stream launches of the commit plan (measured faster than its graph)")},
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
