@@ -25,7 +25,9 @@ constexpr int K_M31 = 16;
 // call is repeated (2^24: 108 us) and lose on fresh inputs (154 us instead of 142).
 constexpr int K_QM31 = 8, K_QM31_STREAM = 10;
 constexpr uint64_t QM31_STREAM = 1ull << 24;
-// 2^26 M31 values: 115 us strided over the grid, 97 here; 2^28 442 / 358.
+// 2^26 M31 values: 115 us strided over the grid, 97 here; 2^28 442 / 358.  In place a column of exactly
+// 256 MB still fits the cache: 2^26 M31 values (2^24 QM31) 91 (107) us through it where the call before
+// left them there, 111 (127) on fresh values, and 98 (117) past it either way, which stays the choice.
 constexpr uint64_t M31_STREAM = 1ull << 26;
 
 template <bool NT>

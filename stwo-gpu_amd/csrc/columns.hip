@@ -226,7 +226,7 @@ __global__ void bitrev_simple_kernel(T* a, uint32_t n, uint32_t log_n) {
 // 2^25 QM31 245 / 262, 2^24 138 / 95.
 constexpr uint32_t BR_STREAM = 27;
 // log of the 4-byte values from which 128 x 128 tiles fill the chip (256 blocks): below, a block that
-// turns a pair of them is the longer chain, and 32 x 32 tiles are faster.  Large / small tiles: 2^16
+// turns a pair of them is the longer chain, and 64 x 64 tiles are faster.  Large / small tiles: 2^16
 // 15.7 / 14.2 us, 2^20 16.6 / 15.1, 2^21 17.1 / 16.3, 2^22 18.7 / 19.5, 2^24 34.9 / 39.9; columns off 16
 // bytes 2^20 17.2 / 15.5, 2^22 19.4 / 21.8.  In 2^14 and 2^15 values no large tile has a partner: 14.0 / 14.1
 // us, off 16 bytes 14.0 / 14.5.

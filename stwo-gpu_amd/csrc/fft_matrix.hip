@@ -7,7 +7,7 @@
 // what four butterfly layers cost, and the passes were bound by exactly those instructions.
 // The matrices are laid out by matrix_kernel from the twiddle tree once per call (17 bytes per
 // domain point and direction, as much as 4 columns), so the passes here serve batches of many
-// columns; see use_matrices for where that starts to pay.
+// columns; see use_matrices_tile and use_matrices_lde for where that starts to pay.
 //
 // Layers 0..3 stay butterflies: their matrices would differ for every 16 values of a column.
 // A thread holds 16 consecutive values there, and its 15 twiddles are seven words: layer 0's
@@ -611,9 +611,15 @@ static void launch_lde(const StridedArgs& S, uint32_t blocks) {
     lde_matrix_kernel<K, false, false><<<blocks, LT, 0, ctx().cur>>>(S);
 }
 
-// From 3 x 2^24 values on, for the same reason: 32 / 48 / 64 / 128 / 256 columns of log 20 at
-// blowup 2 367 / 556 / 725 / 1439 / 2880 us against 370 / 534 / 648 / 1215 / 2300 here, 96 of log
-// 19 534 / 521, 256 of log 18 677 / 657, 512 of log 17 699 / 658; half as many are slower here.
+// From 48 million (2^20) values on, where the matrices' launch is made up for.  Time here / on
+// butterflies (fused schedule) at 32, 48 and 96 million values, blowup 2 | 4 | 8:
+//   log 17   1.05 1.00 0.93 | 1.04 1.00 0.97 | 0.99 0.96 0.95
+//   log 18   1.06 0.99 0.92 | 1.01 0.97 0.94 | 0.94 0.92 0.92
+//   log 19   0.98 0.94 0.88 | 0.98 0.91 0.90 | 0.92 0.89 0.90
+//   log 20   0.96 0.92 0.86 | 0.97 0.91 0.88 | 0.92 0.88 0.86
+// and at 48 million and blowup 32 1.00, 0.95, 0.92, 0.91; the autotuner tries it from half of that.
+// Log 17 to 20 are the sizes whose middle pass is one launch: stage E needs a fifth strided layer,
+// and a ninth would leave its tiles runs of 128 bytes (which cost log 20 1.23 ms instead of 0.98).
 bool use_matrices_lde(uint32_t n, uint32_t log_blowup, uint64_t n_cols) {
   return n >= 17 && n <= 20 && log_blowup >= 1 && (n_cols << n) >= (3ull << 24);
 }
