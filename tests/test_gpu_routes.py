@@ -213,3 +213,22 @@ def test_quotients_of_streamed_columns(log_n, n_cols, n_points):
 def test_quotients_at_the_most_columns(n_cols, matrix):
     """The matrix form's sums are bounded for 8192 columns; one more takes the other form."""
     assert _quotients(4, n_cols, 1, True) == matrix
+
+
+@pytest.mark.parametrize("log_n", [10, 12])
+def test_evaluation_in_place_either_side_of_the_line(log_n):
+    line = (24 << 20) >> log_n
+    coset = S.canonic_half_coset(log_n)
+    tw, _ = S.cached_twiddles(coset)
+    otw, _ = O.precompute_twiddles(coset.initial_index, coset.step_size, coset.log_size)
+    for n_cols, on_matrices in ((line + 1, 1), (line - 1, 0)):
+        cols = _filled(n_cols << log_n, log_n, 1 << log_n)
+        picks = (0, 1, n_cols // 2, n_cols - 2, n_cols - 1)
+        before = [_part(cols, c << log_n, 1 << log_n) for c in picks]
+        logs = np.full(n_cols, log_n, np.uint32).ctypes.data_as(S.u32p)
+        p = _pointers(cols, n_cols, 1 << log_n)
+        with launches("fft_matrices") as got:
+            S.check(S.lib().stwo_hip_evaluate_columns_async(p, logs, p, logs, n_cols, tw, 1 << coset.log_size))
+        assert got["fft_matrices"] == on_matrices
+        for c, v in zip(picks, before):
+            assert (_part(cols, c << log_n, 1 << log_n) == O.evaluate(v, coset.initial_index, otw)).all(), c
